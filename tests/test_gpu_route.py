@@ -168,3 +168,72 @@ def test_routing_feeds_the_layer(cuda_device):
                        w1_scale=wts["w1_scale"], w2_scale=wts["w2_scale"])
     d = (out.float() - out2.float()).abs().max().item()
     assert d <= 2e-2 * out2.float().abs().max().item(), d
+
+
+def _ranked(row, k):
+    """Experts of a row by (value descending, index ascending), NaN and -inf
+    never chosen (0x7fffffff past the last candidate); -0 ties with +0."""
+    c = [e for e in range(len(row)) if row[e] > -np.inf]
+    c.sort(key=lambda e: (-(row[e] + np.float32(0)), e))
+    return (c + [0x7FFFFFFF] * k)[:k]
+
+
+# both sides of every experts-per-lane step of the one-row-per-wave kernel, a
+# narrow row on each side of the row count where it hands over
+@pytest.mark.parametrize("M,E,k", [(5, 1, 1), (9, 64, 32), (9, 65, 8), (9, 128, 8), (9, 129, 8),
+                                   (9, 192, 8), (9, 193, 7), (9, 256, 8), (9, 257, 9), (9, 320, 8),
+                                   (9, 321, 8), (9, 384, 8), (9, 385, 8), (9, 512, 8), (9, 513, 8),
+                                   (9, 768, 8), (9, 769, 8), (9, 1024, 32), (8191, 16, 3),
+                                   (8192, 16, 3)])
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+def test_route_row_edges(cuda_device, M, E, k, dtype):
+    """Ids exact (compared as whole rows, ties included) and weights within
+    rtol 2e-6 (the bar above), with masked experts, rows with fewer candidates
+    than ranks, NaN, infinities and both zeros."""
+    g = torch.Generator().manual_seed(E)
+    x = torch.randint(-6, 7, (M, E), generator=g).float() / 2       # many ties
+    x[1::4, ::2] = float("-inf")
+    x[2, 1:] = float("-inf")                                        # one candidate
+    x[3, E // 2] = float("nan")
+    x[4, :] = torch.where(torch.arange(E) % 2 == 0, -0.0, 0.0)
+    x = x.to(dtype)
+    w, ids = A.fused_topk(torch.empty(M, 1, device=cuda_device), x.to(cuda_device), k, True)
+    xf, gid, gw = x.float().numpy(), _np(ids), _np(w)
+    for r in list(range(min(M, 9))) + [M - 1]:
+        want = _ranked(xf[r], k)
+        assert gid[r].tolist() == want, r
+        v = np.array([xf[r, e] if e < E else -np.inf for e in want], dtype=np.float64)
+        with np.errstate(invalid="ignore"):                         # no candidate at all: NaN
+            p = np.exp(v - v[0])
+        np.testing.assert_allclose(gw[r], p / p.sum(), rtol=2e-6, atol=0)
+
+
+@pytest.mark.parametrize("E,n_group,topk_group", [
+    (64, 1, 1), (64, 32, 5), (128, 2, 1), (192, 4, 2), (256, 16, 16), (320, 8, 3), (384, 8, 4),
+    (512, 32, 9), (768, 4, 3), (1024, 8, 4), (448, 8, 4), (96, 3, 2), (60, 4, 2)])
+@pytest.mark.parametrize("mode", ["softmax", "biased"])
+def test_grouped_forms(cuda_device, E, n_group, topk_group, mode):
+    """Every lanes-per-group form of the one-row-per-wave kernel, and groups
+    that are not whole lanes (the general kernel), against the oracle."""
+    k = min(8, topk_group * (E // n_group))
+    x = _logits(41, E, torch.float32, E + n_group, cuda_device)
+    bias = None
+    if mode == "biased":
+        bias = (torch.randn(E, generator=torch.Generator().manual_seed(E)) * 0.3).to(cuda_device)
+        bias[::5] = float("-inf")                                   # experts switched off
+    w = torch.empty(41, k, dtype=torch.float32, device=cuda_device)
+    ids = torch.empty(41, k, dtype=torch.int32, device=cuda_device)
+    if bias is None:
+        A.grouped_topk(x, w, ids, n_group, topk_group, True, True, 1.5)
+    else:
+        A.biased_grouped_topk(x, bias, w, ids, n_group, topk_group, True, 1.5)
+    if E // n_group < 2:
+        return                                  # a group of one has no second choice to sum
+    if bias is not None and k > 2:
+        k = 2                                   # ranks that every kept group set still fills
+        w, ids = w[:, :k], ids[:, :k]
+        rw, rids = RR.grouped_topk_ref(_np(x), k, n_group, topk_group, False, False, 1.0, _np(bias))
+        assert (_np(ids) == rids).all(axis=1).mean() >= 0.97        # at most one row on a tie
+        return
+    _check_grouped(_np(x), w, ids, k, n_group, topk_group, True, True, 1.5,
+                   None if bias is None else _np(bias))
