@@ -102,6 +102,13 @@ _SIGNATURES = {
         [c_vp, c_int, c_vp, c_vp, c_vp, c_vp, c_vp, c_vp, c_vp, c_vp, c_vp, c_int, c_i64, c_i64,
          c_i64, c_i64, c_i64, c_i64, c_i64, c_i64, c_i64, c_i64, c_vp, c_i64, c_vp],
     ),
+    "aiter_amd_fused_moe_prequant_workspace_bytes": (
+        c_i64, [c_i64, c_i64, c_i64, c_i64, c_i64, c_i64, c_i64]),
+    "aiter_amd_fused_moe_prequant": (
+        c_int,
+        [c_vp, c_vp, c_vp, c_vp, c_vp, c_vp, c_vp, c_vp, c_vp, c_vp, c_vp, c_vp, c_vp, c_int,
+         c_i64, c_i64, c_i64, c_i64, c_i64, c_i64, c_i64, c_i64, c_i64, c_i64, c_vp, c_i64, c_vp],
+    ),
     "aiter_amd_fused_moe_1stage_fp8_blockscale": (
         c_int,
         [c_vp, c_int, c_vp, c_vp, c_vp, c_vp, c_vp, c_vp, c_vp, c_vp, c_vp, c_int, c_i64, c_i64,

@@ -104,10 +104,10 @@ void launch_moe_token_stage2(const uint8_t*, const float*, const uint8_t*, const
                              const uint8_t*, const int32_t*, const float*, void*, int, const void*,
                              int64_t, int64_t, int64_t, int64_t, int, hipStream_t);
 
-// quant.hip: per-pair bf16 rows -> output
-void launch_slot_sum(const uint16_t* part, const int32_t* topk_ids, const int32_t* mask,
-                     int64_t num_experts, const int32_t* num_valid, void* out, int out_dtype,
-                     int64_t rows, int64_t topk, int64_t cols, hipStream_t stream,
+// quant.hip: per-pair bf16 or fp32 rows -> output
+void launch_slot_sum(const void* part, int part_dtype, const int32_t* topk_ids,
+                     const int32_t* mask, int64_t num_experts, const int32_t* num_valid, void* out,
+                     int out_dtype, int64_t rows, int64_t topk, int64_t cols, hipStream_t stream,
                      const void* addend = nullptr);
 
 // moe_route.hip (router top-k)
@@ -127,7 +127,7 @@ void launch_moe_stage1_prefill(const uint8_t*, const float*, int64_t, int64_t, c
                              const float*, int);
 void launch_moe_stage2_prefill(const uint8_t*, const float*, const uint8_t*, const float*,
                                const uint8_t*, const int32_t*, const float*, const int32_t*,
-                               const int32_t*, void*, int, uint16_t*, int64_t, int64_t, int64_t,
+                               const int32_t*, void*, int, void*, int, int64_t, int64_t, int64_t,
                                int64_t, int64_t, int64_t, int64_t, int, hipStream_t, int64_t);
 
 // The 64/128-row kernels (prefill, v2) read their activation operand through
@@ -204,8 +204,8 @@ static bool stage2_on_prefill(int64_t bm, int64_t I, int64_t H, WScale w2s, int6
 }
 
 // acc: [tokens, H] accumulated atomically, fp32 or (the reference's moe_buf)
-// bf16 / fp16 by acc_dtype; part (prefill kernel only): bf16 [pairs, H] rows
-// written once each, acc unused.
+// bf16 / fp16 by acc_dtype; part (prefill kernel only): [pairs, H] rows of
+// part_dtype (bf16 or fp32) written once each, acc unused.
 // est_pairs: the pairs expected on this GPU (the EP share's fraction of
 // tokens * topk when the caller knows it), a launch-shape hint only.
 static void stage2_dispatch(const uint8_t* a2, const float* a2s, const uint8_t* w2,
@@ -213,7 +213,8 @@ static void stage2_dispatch(const uint8_t* a2, const float* a2s, const uint8_t* 
                             const int32_t* seid, const int32_t* nv, void* acc, int acc_dtype,
                             int64_t a_rows, int64_t I, int64_t H, int64_t E, int64_t topk,
                             int64_t bm, int64_t mblocks, int sh, hipStream_t s,
-                            uint16_t* part = nullptr, int64_t est_pairs = -1) {
+                            void* part = nullptr, int part_dtype = DT_BF16,
+                            int64_t est_pairs = -1) {
     const bool on_prefill = stage2_on_prefill(bm, I, H, w2s, a_rows, E, est_pairs);
     AMD_CHECK(!part || on_prefill, "per-pair rows need the prefill kernel");
     if (stream_supported(bm, I) && H % 256 == 0)
@@ -221,8 +222,8 @@ static void stage2_dispatch(const uint8_t* a2, const float* a2s, const uint8_t* 
                                  acc_dtype, a_rows, I, H, E, topk, bm, mblocks, sh, s);
     else if (on_prefill)
         launch_moe_stage2_prefill(a2, a2s, w2, w2s.f32, w2s.e8m0, sid, sw, seid, nv, acc,
-                                  acc_dtype, part, a_rows, I, H, E, topk, bm, mblocks, sh, s,
-                                  est_pairs < 0 ? a_rows : est_pairs);
+                                  acc_dtype, part, part_dtype, a_rows, I, H, E, topk, bm, mblocks,
+                                  sh, s, est_pairs < 0 ? a_rows : est_pairs);
     else if (v2_supported(bm, I) && H % 256 == 0 && a_fits32(a_rows, I))
         launch_moe_stage2_fp8bs_v2(a2, a2s, w2, w2s.f32, w2s.e8m0, sid, sw, seid, nv, acc,
                                    acc_dtype, a_rows, I, H, E, topk, bm, mblocks, sh, s);
@@ -308,10 +309,22 @@ struct FusedLayout {
 
 int64_t align256(int64_t x) { return (x + 255) & ~int64_t(255); }
 
+// Layers that sum in fp32 throughout (see fused_entry): per-pair fp32 rows
+// written and read once, or fp32 atomics, which go past the XCDs' L2s and meet
+// on a token's row. Layer times on MI355X, hidden 4096, top-8, atomics / rows:
+// 16 experts of inter 1536 T=256 163 / 152 us, T=1500 429 / 394, T=8192 2030 /
+// 1900; 32 of 256 experts of inter 2048 T=2048 213 / 195, T=8192 397 / 361; all
+// 256 T=600 1231 / 1252, T=2048 1414 / 1433, T=8192 2907 / 2878. Beyond this
+// many bytes of rows the workspace would outgrow the layer's other sections,
+// so larger layers keep the accumulator.
+constexpr int64_t kMaxF32RowBytes = int64_t(1) << 30;
+
+bool f32_rows_fit(int64_t T, int64_t k, int64_t H) { return T * k * H * 4 <= kMaxF32RowBytes; }
+
 // E_local: the experts this GPU holds (E_sort: the ids' range, global under
-// an expert mask).
+// an expert mask). sum32: the layer sums in fp32 throughout.
 FusedLayout fused_layout(int64_t T, int64_t H, int64_t I, int64_t E_sort, int64_t E_local,
-                         int64_t k, int64_t bm) {
+                         int64_t k, int64_t bm, bool sum32 = false) {
     FusedLayout L;
     L.cap = sorted_capacity_for(T, k, E_sort, bm);
     L.blocks = ceil_div(L.cap, bm);
@@ -332,9 +345,10 @@ FusedLayout fused_layout(int64_t T, int64_t H, int64_t I, int64_t E_sort, int64_
     L.off_a1_scale = o;    o = align256(o + T * (H / 128) * 4);
     L.off_a2 = o;          o = align256(o + T * k * I);
     L.off_a2_scale = o;    o = align256(o + T * k * (I / 128) * 4);
-    // fp32 accumulator [T, H], or per-pair bf16 rows [T*k, H] when stage 2
-    // runs on the prefill kernel: room for either
-    L.off_acc = o;         o = align256(o + std::max(T * H * 4, T * k * H * 2));
+    // fp32 accumulator [T, H], or per-pair rows [T*k, H] when stage 2 runs on
+    // the prefill kernel: room for either
+    const int64_t row_bytes = !sum32 ? 2 : f32_rows_fit(T, k, H) ? 4 : 0;
+    L.off_acc = o;         o = align256(o + std::max(T * H * 4, T * k * H * row_bytes));
     L.kcnt_bytes = L.ksplit > 1 ? align256(L.kmb * (I / 128) * 4) : 0;
     L.off_kcnt = o;        o += L.kcnt_bytes;
     L.off_kpart = o;       o = align256(o + stream_ksplit_part_bytes(bm, L.kmb, I, L.ksplit));
@@ -504,7 +518,9 @@ struct PreQuant {
 };
 
 // accumulate: the layer is added to out's previous contents (rounded once
-// from fp32) instead of replacing them.
+// from fp32) instead of replacing them. sum32: each pair's weighted row stays
+// in fp32 until a token's rows are summed (the stage-wise calls' precision);
+// otherwise the prefill kernel rounds it to bf16 first.
 void fused_entry(const void* hidden_states, int hidden_dtype, const void* w1, WScale w1s,
                  const void* w2, WScale w2s, const float* topk_weights, const int32_t* topk_ids,
                  const int32_t* expert_mask, const int32_t* num_local_tokens, void* out,
@@ -512,7 +528,7 @@ void fused_entry(const void* hidden_states, int hidden_dtype, const void* w1, WS
                  int64_t num_experts, int64_t global_experts, int64_t topk, int64_t block_m,
                  int64_t activation, int64_t doweight_stage1, int64_t w_shuffled,
                  void* workspace, int64_t workspace_bytes, void* stream, bool one_launch = false,
-                 PreQuant pre = PreQuant{}, bool accumulate = false) {
+                 PreQuant pre = PreQuant{}, bool accumulate = false, bool sum32 = false) {
     check_dims(model_dim, inter_dim);
     AMD_CHECK(activation == kActSilu || activation == kActGelu,
               "only ActivationType.Silu (0) and Gelu (1) are supported, got " +
@@ -544,7 +560,7 @@ void fused_entry(const void* hidden_states, int hidden_dtype, const void* w1, WS
     check_ptr(out, "out");
     AMD_CHECK(topk_weights && topk_ids, "a required pointer is NULL");
     const FusedLayout L =
-        fused_layout(tokens, model_dim, inter_dim, E_sort, num_experts, topk, block_m);
+        fused_layout(tokens, model_dim, inter_dim, E_sort, num_experts, topk, block_m, sum32);
     AMD_CHECK(workspace_bytes >= L.total, "workspace of " + std::to_string(L.total) +
                                               " bytes required, got " +
                                               std::to_string(workspace_bytes));
@@ -562,13 +578,15 @@ void fused_entry(const void* hidden_states, int hidden_dtype, const void* w1, WS
     uint8_t* a2 = ws + L.off_a2;
     float* a2_scale = reinterpret_cast<float*>(ws + L.off_a2_scale);
     float* acc = reinterpret_cast<float*>(ws + L.off_acc);
-    // stage 2 on the prefill kernel writes each pair's weighted row once (bf16)
-    // and one pass sums a token's slots: no fp32 atomics, no accumulator to clear
+    // stage 2 on the prefill kernel writes each pair's weighted row once and
+    // one pass sums a token's slots: no fp32 atomics, no accumulator to clear
     // pairs expected on this GPU (the expert-parallel share of tokens * topk)
     const int64_t local_pairs = tokens * topk * num_experts / E_sort;
-    uint16_t* part = stage2_on_prefill(block_m, inter_dim, model_dim, w2s, tokens * topk,
-                                       num_experts, local_pairs)
-                         ? reinterpret_cast<uint16_t*>(ws + L.off_acc) : nullptr;
+    const int part_dtype = sum32 ? DT_FP32 : DT_BF16;
+    void* part = stage2_on_prefill(block_m, inter_dim, model_dim, w2s, tokens * topk, num_experts,
+                                   local_pairs) &&
+                         (!sum32 || f32_rows_fit(tokens, topk, model_dim))
+                     ? ws + L.off_acc : nullptr;
     hipStream_t s = (hipStream_t)stream;
     timing_mark(0, s);
     const int sh = (int)(w_shuffled != 0);
@@ -637,11 +655,11 @@ void fused_entry(const void* hidden_states, int hidden_dtype, const void* w1, WS
     stage2_dispatch(a2, a2_scale, (const uint8_t*)w2, w2s, sorted_ids, dw ? nullptr : sorted_w,
                     sorted_eids,
                     num_valid, part ? nullptr : acc, DT_FP32, tokens * topk, inter_dim, model_dim,
-                    num_experts, topk, block_m, L.blocks, sh, s, part, local_pairs);
+                    num_experts, topk, block_m, L.blocks, sh, s, part, part_dtype, local_pairs);
     timing_mark(4, s);
     if (part)
-        launch_slot_sum(part, topk_ids, expert_mask, E_sort, num_valid, out, out_dtype, tokens,
-                        topk, model_dim, s, addend);
+        launch_slot_sum(part, part_dtype, topk_ids, expert_mask, E_sort, num_valid, out, out_dtype,
+                        tokens, topk, model_dim, s, addend);
     else
         launch_acc_to_out(acc, out, out_dtype, num_valid, tokens, model_dim, s, addend);
     timing_mark(5, s);
@@ -1002,6 +1020,51 @@ int aiter_amd_fused_moe_a8w4(const void* hidden_states, int hidden_dtype, const 
                     num_local_tokens, out, out_dtype, tokens, model_dim, inter_dim, num_experts,
                     global_experts, topk, block_m, activation, doweight_stage1, w_shuffled, workspace,
                     workspace_bytes, stream);
+    });
+}
+
+int64_t aiter_amd_fused_moe_prequant_workspace_bytes(int64_t tokens, int64_t model_dim,
+                                                     int64_t inter_dim, int64_t num_experts,
+                                                     int64_t global_experts, int64_t topk,
+                                                     int64_t block_m) {
+    if (tokens < 0 || model_dim <= 0 || inter_dim <= 0 || num_experts < 1 ||
+        global_experts < num_experts || topk < 1)
+        return -1;
+    if (block_m <= 0)
+        block_m = default_block_m(tokens, topk, num_experts, global_experts, model_dim, inter_dim);
+    return fused_layout(tokens, model_dim, inter_dim, global_experts, num_experts, topk, block_m,
+                        true).total;
+}
+
+int aiter_amd_fused_moe_prequant(
+    const void* a1, const float* a1_scale, const void* w1, const float* w1_scale,
+    const uint8_t* w1_scale_e8m0, const void* w2, const float* w2_scale,
+    const uint8_t* w2_scale_e8m0, const float* topk_weights, const int32_t* topk_ids,
+    const int32_t* expert_mask, const int32_t* num_local_tokens, void* out, int out_dtype,
+    int64_t tokens, int64_t model_dim, int64_t inter_dim, int64_t num_experts,
+    int64_t global_experts, int64_t topk, int64_t block_m, int64_t activation,
+    int64_t doweight_stage1, int64_t w_shuffled, void* workspace, int64_t workspace_bytes,
+    void* stream) {
+    return safe_call([&] {
+        AMD_CHECK((w1_scale != nullptr) != (w1_scale_e8m0 != nullptr) &&
+                      (w1_scale != nullptr) == (w2_scale != nullptr) &&
+                      (w1_scale_e8m0 != nullptr) == (w2_scale_e8m0 != nullptr),
+                  "give both fp32 block scales (fp8 weights) or both e8m0 scales (MXFP4)");
+        if (w1_scale_e8m0) {
+            check_e8m0(w1_scale_e8m0, "w1_scale");
+            check_e8m0(w2_scale_e8m0, "w2_scale");
+        }
+        check_ptr(a1, "a1");
+        PreQuant pre;
+        pre.a1 = (const uint8_t*)a1;
+        pre.a1_scale = a1_scale;
+        pre.sa_row = model_dim / 128;
+        pre.sa_kb = 1;
+        fused_entry(nullptr, DT_FP8, w1, WScale{w1_scale, w1_scale_e8m0}, w2,
+                    WScale{w2_scale, w2_scale_e8m0}, topk_weights, topk_ids, expert_mask,
+                    num_local_tokens, out, out_dtype, tokens, model_dim, inter_dim, num_experts,
+                    global_experts, topk, block_m, activation, doweight_stage1, w_shuffled,
+                    workspace, workspace_bytes, stream, false, pre, false, true);
     });
 }
 

@@ -38,6 +38,7 @@
 // paid once; the next tile's first loads are in flight during a tile's
 // epilogue).
 #include <cstdlib>
+#include <type_traits>
 
 #include "common.h"
 
@@ -66,7 +67,8 @@ struct Args {
     float* a2_scale;
     void* acc;                 // stage 2 out [T, N]: fp32, bf16 or fp16 (acc_dtype)
     int acc_dtype;
-    uint16_t* part;            // stage 2: bf16 rows [pairs, N] instead of acc (or NULL)
+    void* part;                // stage 2: rows [pairs, N] instead of acc (or NULL), bf16 or
+    int part_dtype;            // (256-column tiles) fp32
     int K;
     int N;                     // weight rows per expert
     int inter;
@@ -623,7 +625,9 @@ __global__ __launch_bounds__(kThreads, 2) void moe_gemm_prefill_kernel(Args g) {
                 // was the final K step (an FP8 tile's 64 rows in one pass; four
                 // through an A stage took T=8192 924-928 us against 917-921), the
                 // 128-column tile through the free A stage
-                auto stage_rows = [&](uint16_t* s_p, auto rpp, auto pw) __attribute__((always_inline)) {
+                auto stage_rows = [&](auto* s_p, auto rpp, auto pw) __attribute__((always_inline)) {
+                    using TP = std::remove_pointer_t<decltype(s_p)>;
+                    constexpr int EPP = 16 / sizeof(TP);      // elements per 16-byte piece
                     constexpr int RPP = decltype(rpp)::value;
                     constexpr int PW = decltype(pw)::value;   // staged row pitch (elements)
                     static_assert(RPP % 16 == 0 && BM % RPP == 0,
@@ -639,26 +643,38 @@ __global__ __launch_bounds__(kThreads, 2) void moe_gemm_prefill_kernel(Args g) {
                                 const float wgt = s_w[row];
                                 const int lrow = row - hf * RPP;
 #pragma unroll
-                                for (int ct = 0; ct < NCT; ++ct)
-                                    s_p[lrow * PW + wn * NCT * 16 + ct * 16 + lr] =
-                                        f32_to_bf16_bits(acc[rt][ct][v] * wgt);
+                                for (int ct = 0; ct < NCT; ++ct) {
+                                    const float y = acc[rt][ct][v] * wgt;
+                                    TP* d = s_p + lrow * PW + wn * NCT * 16 + ct * 16 + lr;
+                                    if constexpr (sizeof(TP) == 4)
+                                        *d = y;
+                                    else
+                                        *d = f32_to_bf16_bits(y);
+                                }
                             }
                         }
                         __syncthreads();
-                        for (int q = tid; q < RPP * (NW / 8); q += kThreads) {
-                            const int lrow = q / (NW / 8), piece = q % (NW / 8);
+                        for (int q = tid; q < RPP * (NW / EPP); q += kThreads) {
+                            const int lrow = q / (NW / EPP), piece = q % (NW / EPP);
                             const int64_t pair = s_arow[lrow + hf * RPP];
                             if (pair < 0) continue;
-                            *reinterpret_cast<v4i*>(g.part + pair * g.N + nc + piece * 8) =
-                                *reinterpret_cast<const v4i*>(s_p + lrow * PW + piece * 8);
+                            *reinterpret_cast<v4i*>(reinterpret_cast<TP*>(g.part) + pair * g.N +
+                                                    nc + piece * EPP) =
+                                *reinterpret_cast<const v4i*>(s_p + lrow * PW + piece * EPP);
                         }
                         __syncthreads();
                     }
                 };
                 constexpr int A_ROWS = A_BYTES / (NW * 2);
-                if constexpr (NW2 > 128)
-                    stage_rows(reinterpret_cast<uint16_t*>(s_sc), IntC<SC_RPP>{}, IntC<SC_PW>{});
-                else
+                if constexpr (NW2 > 128) {
+                    // fp32 rows at a pitch of NW + 4 (rows 4 apart start 16 banks
+                    // apart), as many per pass as the same buffer holds
+                    if (g.part_dtype == DT_FP32)
+                        stage_rows(s_sc, IntC<SC_FLOATS / (NW + 4) / 16 * 16>{}, IntC<NW + 4>{});
+                    else
+                        stage_rows(reinterpret_cast<uint16_t*>(s_sc), IntC<SC_RPP>{},
+                                   IntC<SC_PW>{});
+                } else
                     stage_rows(reinterpret_cast<uint16_t*>(&s_a[stg][0]),
                                IntC<(A_ROWS >= BM ? BM : A_ROWS)>{}, IntC<NW>{});
             } else {
@@ -1089,9 +1105,10 @@ void launch_moe_stage2_prefill(const uint8_t* a2, const float* a2_scale, const u
                                const float* w2_scale, const uint8_t* w2_scale_e8m0,
                                const int32_t* sorted_ids, const float* sorted_w,
                                const int32_t* sorted_eids, const int32_t* num_valid, void* acc, int acc_dtype,
-                               uint16_t* part, int64_t a_rows, int64_t inter, int64_t hidden,
-                               int64_t E, int64_t topk, int64_t block_m, int64_t max_m_blocks,
-                               int shuffled, hipStream_t stream, int64_t est_pairs) {
+                               void* part, int part_dtype, int64_t a_rows, int64_t inter,
+                               int64_t hidden, int64_t E, int64_t topk, int64_t block_m,
+                               int64_t max_m_blocks, int shuffled, hipStream_t stream,
+                               int64_t est_pairs) {
     pf::Args g{};
     g.a = a2;
     g.a_scale = a2_scale;
@@ -1107,13 +1124,14 @@ void launch_moe_stage2_prefill(const uint8_t* a2, const float* a2_scale, const u
     g.acc = acc;
     g.acc_dtype = acc_dtype;
     g.part = part;
+    g.part_dtype = part_dtype;
     g.K = (int)inter;
     g.N = (int)hidden;
     g.inter = (int)inter;
     g.topk = (int)topk;
     g.E = (int)E;
     g.a_rows = a_rows;
-    const bool wide = pf::pick_wide2(hidden);
+    const bool wide = pf::pick_wide2(hidden) || (part && part_dtype == DT_FP32);
     const int rows = wide ? 64 : (int)block_m;
     g.n_tiles = (int)(hidden / (wide ? 256 : 128));
     g.block_m = (int)block_m;

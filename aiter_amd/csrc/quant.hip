@@ -124,18 +124,48 @@ void launch_acc_to_out(const float* acc, void* out, int out_dtype, const int32_t
     AMD_HIP_CHECK(hipGetLastError());
 }
 
-// ------------------------------------ per-pair bf16 rows -> output ---
+// ---------------------------- per-pair bf16 or fp32 rows -> output ---
 // out[t, :] = round(sum over the token's routed slots j of part[t*topk + j, :])
 // for t < tokens (= *num_valid[1]), summed in fp32 in slot order. A slot is
 // routed when sorting kept its pair: expert id in [0, num_experts) and, with
 // an expert mask, mask[id] != 0. topk <= 32. The token's valid slots are
 // checked once (lane j checks slot j; a ballot gives the bit mask).
 //
+// Rows in fp32 (layers whose sums stay in 32 bits until the output's rounding)
+// take two 16-byte loads per 8 columns.
+template <typename TP>
+struct Row8 {
+    static constexpr int kPieces = sizeof(TP) / 2;      // 16-byte loads per 8 columns
+    v4i v[kPieces];
+
+    __device__ __forceinline__ void clear() {
+#pragma unroll
+        for (int p = 0; p < kPieces; ++p) v[p] = v4i{0, 0, 0, 0};
+    }
+    __device__ __forceinline__ void load(const TP* src) {
+#pragma unroll
+        for (int p = 0; p < kPieces; ++p)
+            v[p] = __builtin_nontemporal_load(reinterpret_cast<const v4i*>(src) + p);
+    }
+    __device__ __forceinline__ void add_to(float (&a)[8]) const {
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+            if constexpr (kPieces == 1) {
+                a[2 * e] += bf16_bits_to_f32((uint16_t)((uint32_t)v[0][e] & 0xFFFFu));
+                a[2 * e + 1] += bf16_bits_to_f32((uint16_t)((uint32_t)v[0][e] >> 16));
+            } else {
+                a[e] += __builtin_bit_cast(float, (int)v[0][e]);
+                a[4 + e] += __builtin_bit_cast(float, (int)v[kPieces - 1][e]);
+            }
+        }
+    }
+};
+
 // slot_sum_kernel: one token per workgroup; each lane sums two 8-column
 // pieces of a 4096-column row in one pass, the loads of 8 slots of both
 // pieces in flight before any sum.
-template <bool kBf16>
-__global__ __launch_bounds__(256) void slot_sum_kernel(const uint16_t* __restrict__ part,
+template <bool kBf16, typename TP>
+__global__ __launch_bounds__(256) void slot_sum_kernel(const TP* __restrict__ part,
                                                        const int32_t* __restrict__ topk_ids,
                                                        const int32_t* __restrict__ mask,
                                                        int num_experts,
@@ -156,33 +186,27 @@ __global__ __launch_bounds__(256) void slot_sum_kernel(const uint16_t* __restric
             ok = id >= 0 && id < num_experts && (!mask || mask[id] != 0);
         }
         const uint32_t valid = (uint32_t)__builtin_amdgcn_ballot_w64(ok);
-        const uint16_t* src = part + t * topk * (int64_t)cols;
+        const TP* src = part + t * topk * (int64_t)cols;
         for (int c0 = tl; c0 < c8; c0 += 2 * kSpan) {
             const int cc[2] = {c0, c0 + kSpan};
             float a[2][8] = {};
             for (int j0 = 0; j0 < topk; j0 += 8) {
-                v4i v[2][8];
+                Row8<TP> v[2][8];
 #pragma unroll
                 for (int h = 0; h < 2; ++h)
 #pragma unroll
                     for (int u = 0; u < 8; ++u) {
                         const int j = j0 + u;
-                        v[h][u] = v4i{0, 0, 0, 0};
+                        v[h][u].clear();
                         if (cc[h] < c8 && j < topk && ((valid >> j) & 1u))
-                            v[h][u] = __builtin_nontemporal_load(reinterpret_cast<const v4i*>(
-                                src + (int64_t)j * cols + cc[h] * 8));
+                            v[h][u].load(src + (int64_t)j * cols + cc[h] * 8);
                     }
 #pragma unroll
                 for (int h = 0; h < 2; ++h)
 #pragma unroll
                     for (int u = 0; u < 8; ++u) {
                         const int j = j0 + u;
-                        if (j >= topk || !((valid >> j) & 1u)) continue;
-#pragma unroll
-                        for (int e = 0; e < 4; ++e) {
-                            a[h][2 * e] += bf16_bits_to_f32((uint16_t)((uint32_t)v[h][u][e] & 0xFFFFu));
-                            a[h][2 * e + 1] += bf16_bits_to_f32((uint16_t)((uint32_t)v[h][u][e] >> 16));
-                        }
+                        if (j < topk && ((valid >> j) & 1u)) v[h][u].add_to(a[h]);
                     }
             }
 #pragma unroll
@@ -211,12 +235,12 @@ __global__ __launch_bounds__(256) void slot_sum_kernel(const uint16_t* __restric
 // EP share (32 of 256 experts, 64-row blocks): T=4096 20.0 -> 18.9 us, T=2048
 // 14.7 -> 13.7 us against two pieces per pass (the per-workgroup kernel took
 // 21 us); 4 pieces per lane (two passes, 92 instead of 168 VGPRs) 20.5 us.
-template <bool kBf16>
+template <bool kBf16, typename TP>
 __global__ __launch_bounds__(256) void slot_sum_wave_kernel(
-    const uint16_t* __restrict__ part, const int32_t* __restrict__ topk_ids,
+    const TP* __restrict__ part, const int32_t* __restrict__ topk_ids,
     const int32_t* __restrict__ mask, int num_experts, const int32_t* __restrict__ num_valid,
     uint16_t* out, int64_t rows, int topk, int cols, const uint16_t* addend) {
-    constexpr int kPieces = 8;
+    constexpr int kPieces = 16 / sizeof(TP);             // 4 of fp32 rows: the same bytes in flight
     int64_t tokens = (int64_t)num_valid[1];
     tokens = tokens < rows ? tokens : rows;
     const int c8 = cols / 8;
@@ -229,29 +253,22 @@ __global__ __launch_bounds__(256) void slot_sum_wave_kernel(
             ok = id >= 0 && id < num_experts && (!mask || mask[id] != 0);
         }
         const uint32_t valid = (uint32_t)__builtin_amdgcn_ballot_w64(ok);
-        const uint16_t* src = part + t * topk * (int64_t)cols;
+        const TP* src = part + t * topk * (int64_t)cols;
         for (int base = lane; base < c8; base += 64 * kPieces) {
             float a[kPieces][8] = {};
             uint32_t m = valid;
             while (m != 0) {
                 const int j = __builtin_ctz(m);
                 m &= m - 1;
-                v4i v[kPieces];
+                Row8<TP> v[kPieces];
 #pragma unroll
                 for (int i = 0; i < kPieces; ++i) {
                     const int cc = base + 64 * i;
-                    v[i] = v4i{0, 0, 0, 0};
-                    if (cc < c8)
-                        v[i] = __builtin_nontemporal_load(
-                            reinterpret_cast<const v4i*>(src + (int64_t)j * cols + cc * 8));
+                    v[i].clear();
+                    if (cc < c8) v[i].load(src + (int64_t)j * cols + cc * 8);
                 }
 #pragma unroll
-                for (int i = 0; i < kPieces; ++i)
-#pragma unroll
-                    for (int e = 0; e < 4; ++e) {
-                        a[i][2 * e] += bf16_bits_to_f32((uint16_t)((uint32_t)v[i][e] & 0xFFFFu));
-                        a[i][2 * e + 1] += bf16_bits_to_f32((uint16_t)((uint32_t)v[i][e] >> 16));
-                    }
+                for (int i = 0; i < kPieces; ++i) v[i].add_to(a[i]);
             }
 #pragma unroll
             for (int i = 0; i < kPieces; ++i) {
@@ -272,23 +289,31 @@ __global__ __launch_bounds__(256) void slot_sum_wave_kernel(
     }
 }
 
-void launch_slot_sum(const uint16_t* part, const int32_t* topk_ids, const int32_t* mask,
-                     int64_t num_experts, const int32_t* num_valid, void* out, int out_dtype,
-                     int64_t rows, int64_t topk, int64_t cols, hipStream_t stream,
+void launch_slot_sum(const void* part, int part_dtype, const int32_t* topk_ids,
+                     const int32_t* mask, int64_t num_experts, const int32_t* num_valid, void* out,
+                     int out_dtype, int64_t rows, int64_t topk, int64_t cols, hipStream_t stream,
                      const void* addend) {
     if (rows == 0 || cols == 0) return;
     // an expert mask means an expert-parallel share: most slots are not routed here
     const bool per_wave = mask != nullptr;
     const int blocks = (int)std::min<int64_t>(ceil_div(rows, per_wave ? 4 : 1), 8192);
-    auto go = [&](auto kern) {
-        hipLaunchKernelGGL(kern, dim3(blocks), dim3(256), 0, stream, part, topk_ids, mask,
+    auto go = [&](auto kern, auto* rows_of_pairs) {
+        hipLaunchKernelGGL(kern, dim3(blocks), dim3(256), 0, stream, rows_of_pairs, topk_ids, mask,
                            (int)num_experts, num_valid, (uint16_t*)out, rows, (int)topk,
                            (int)cols, (const uint16_t*)addend);
     };
-    if (out_dtype == DT_BF16)
-        per_wave ? go(slot_sum_wave_kernel<true>) : go(slot_sum_kernel<true>);
+    auto with_rows = [&](auto* rp) {
+        using TP = std::remove_const_t<std::remove_pointer_t<decltype(rp)>>;
+        if (out_dtype == DT_BF16)
+            per_wave ? go(slot_sum_wave_kernel<true, TP>, rp) : go(slot_sum_kernel<true, TP>, rp);
+        else
+            per_wave ? go(slot_sum_wave_kernel<false, TP>, rp)
+                     : go(slot_sum_kernel<false, TP>, rp);
+    };
+    if (part_dtype == DT_FP32)
+        with_rows(reinterpret_cast<const float*>(part));
     else
-        per_wave ? go(slot_sum_wave_kernel<false>) : go(slot_sum_kernel<false>);
+        with_rows(reinterpret_cast<const uint16_t*>(part));
     AMD_HIP_CHECK(hipGetLastError());
 }
 

@@ -43,19 +43,20 @@ def _stream(dev: torch.device) -> int:
 
 
 def _layer_workspace_bytes(M: int, model_dim: int, inter_dim: int, E: int, global_E: int,
-                           topk: int, block_m: int) -> int:
+                           topk: int, block_m: int,
+                           entry: str = "aiter_amd_fused_moe_workspace_bytes") -> int:
     # AITER_AMD_ST_KSPLIT1 (the stage-1 K-split override) sizes the split's
     # partial sums and AITER_AMD_SORT_CT (the sorting chunk override) the
     # sorting's chunk counts, so their values are part of the cached query's key
-    return _workspace_query(M, model_dim, inter_dim, E, global_E, topk, block_m,
+    return _workspace_query(entry, M, model_dim, inter_dim, E, global_E, topk, block_m,
                             os.environ.get("AITER_AMD_ST_KSPLIT1"),
                             os.environ.get("AITER_AMD_SORT_CT"))
 
 
 @functools.lru_cache(maxsize=1024)
-def _workspace_query(M, model_dim, inter_dim, E, global_E, topk, block_m, ksplit_env, ct_env):
-    return _abi.query("aiter_amd_fused_moe_workspace_bytes", M, model_dim, inter_dim, E,
-                      global_E, topk, block_m)
+def _workspace_query(entry, M, model_dim, inter_dim, E, global_E, topk, block_m, ksplit_env,
+                     ct_env):
+    return _abi.query(entry, M, model_dim, inter_dim, E, global_E, topk, block_m)
 
 
 @functools.lru_cache(maxsize=16)
@@ -483,21 +484,20 @@ def _fused_moe_impl(hidden_states, w1, w2, topk_weight, topk_ids, expert_mask, a
             int(shuffled), ws.data_ptr(), ws_bytes, stream)
         return out
 
-    # fp8 activations with caller-provided 1x128 scales: skip the quant step
-    sorted_ids, sorted_w, sorted_eids, num_valid, acc = moe_sorting(
-        topk_ids, topk_weight, global_E, model_dim, dtypes.fp32, block_m, mask,
-        num_local_tokens, moe_sorting_dispatch_policy)
-    st1 = moe_stage1_a8w4 if a8w4 else moe_stage1_fp8_blockscale
-    st2 = moe_stage2_a8w4 if a8w4 else moe_stage2_fp8_blockscale
-    # doweight_stage1: the routing weights go to stage 1, stage 2 sums unweighted
-    # (aiter/fused_moe.py:1253, 1330)
-    a2, a2s = st1(hidden_states.contiguous(), a1_scale.contiguous(), w1c, w1s, sorted_ids,
-                  sorted_eids, num_valid, topk, block_m, shuffled,
-                  sorted_weights=sorted_w if doweight_stage1 else None, activation=activation)
-    st2(a2, a2s, w2c, w2s, sorted_ids, None if doweight_stage1 else sorted_w, sorted_eids,
-        num_valid, acc, block_m, shuffled)
-    _abi.call("aiter_amd_moe_acc_to_out", acc.data_ptr(), out.data_ptr(), AITER_DTYPE[out_dtype],
-              num_valid.data_ptr(), M, model_dim, stream)
+    # fp8 activations with caller-provided 1x128 scales: no quant step, and a
+    # token's weighted rows are summed in fp32
+    a1, a1s = hidden_states.contiguous(), a1_scale.contiguous()
+    ws_bytes = _layer_workspace_bytes(M, model_dim, inter_dim, E, global_E, topk, block_m,
+                                      "aiter_amd_fused_moe_prequant_workspace_bytes")
+    ws = torch.empty(ws_bytes, dtype=torch.uint8, device=device)
+    s1, s2 = w1s.data_ptr(), w2s.data_ptr()
+    _abi.call(
+        "aiter_amd_fused_moe_prequant", a1.data_ptr(), a1s.data_ptr(), w1c.data_ptr(),
+        None if a8w4 else s1, s1 if a8w4 else None, w2c.data_ptr(), None if a8w4 else s2,
+        s2 if a8w4 else None, topk_weight.data_ptr(), topk_ids.data_ptr(), _ptr(mask),
+        _ptr(num_local_tokens), out.data_ptr(), AITER_DTYPE[out_dtype], M, model_dim, inter_dim,
+        E, global_E, topk, block_m, int(activation), int(bool(doweight_stage1)), int(shuffled),
+        ws.data_ptr(), ws_bytes, stream)
     return out
 
 

@@ -317,6 +317,31 @@ int aiter_amd_fused_moe_a8w4(const void* hidden_states, int hidden_dtype, const 
                              int64_t doweight_stage1, int64_t w_shuffled, void* workspace,
                              int64_t workspace_bytes, void* stream);
 
+/* Bytes of workspace for aiter_amd_fused_moe_prequant; arguments as
+ * aiter_amd_fused_moe_workspace_bytes. */
+int64_t aiter_amd_fused_moe_prequant_workspace_bytes(int64_t tokens, int64_t model_dim,
+                                                     int64_t inter_dim, int64_t num_experts,
+                                                     int64_t global_experts, int64_t topk,
+                                                     int64_t block_m);
+
+/* The whole 2-stage layer on activations that are already fp8: fused_moe_
+ * with fp8 hidden_states and a1_scale (aiter/fused_moe.py:256-265), which the
+ * reference runs as moe_sorting and the two stage calls.
+ *   a1 [tokens, model_dim] fp8, a1_scale [tokens, model_dim/128] f32; weights
+ *   fp8 with w1_scale / w2_scale, or MXFP4 with the e8m0 pair (the other pair
+ *   NULL); everything else as aiter_amd_fused_moe_fp8_blockscale. A token's
+ *   weighted rows are summed in fp32 and rounded once, as the stage calls
+ *   with an fp32 out_acc do. */
+int aiter_amd_fused_moe_prequant(
+    const void* a1, const float* a1_scale, const void* w1, const float* w1_scale,
+    const uint8_t* w1_scale_e8m0, const void* w2, const float* w2_scale,
+    const uint8_t* w2_scale_e8m0, const float* topk_weights, const int32_t* topk_ids,
+    const int32_t* expert_mask, const int32_t* num_local_tokens, void* out, int out_dtype,
+    int64_t tokens, int64_t model_dim, int64_t inter_dim, int64_t num_experts,
+    int64_t global_experts, int64_t topk, int64_t block_m, int64_t activation,
+    int64_t doweight_stage1, int64_t w_shuffled, void* workspace, int64_t workspace_bytes,
+    void* stream);
+
 /* The whole layer with both GEMMs in ONE launch; replaces fused_moe_1stage
  * -> fmoe_fp8_blockscale_g1u1 (aiter/fused_moe.py:367-511,
  * csrc/py_itfs_cu/asm_fmoe.cu:858-922), which the reference picks per shape

@@ -1007,3 +1007,64 @@ def test_fused_moe_direct_hip_graph_replay(cuda_device, monkeypatch, shape):
         eager = run(x).float()
         torch.cuda.synchronize()
         assert torch.count_nonzero(got).item() > 0 and torch.equal(got, eager), f"replay {i}"
+
+
+@pytest.mark.parametrize("weights", ["fp8", "mxfp4"])
+@pytest.mark.parametrize("tokens,bm,variant", [
+    (1, 16, "plain"), (17, 16, "plain"), (65, 32, "plain"), (63, 64, "plain"), (300, 64, "plain"),
+    (300, 128, "plain"), (300, 64, "mask"), (300, 64, "local_tokens"), (300, 128, "doweight"),
+    (300, None, "fp16")])
+def test_prequant_layer_matches_stage_calls(cuda_device, weights, tokens, bm, variant):
+    """fp8 activations through the one-call entry against the stage calls with
+    an fp32 accumulator. Both run the same stage-1 kernel and sum a token's
+    rows in fp32, in another order, then round once: outputs differ by at most
+    one 16-bit step (2^-8 relative for bf16), or by topk * 2^-23 of the largest
+    sum where terms cancel."""
+    cfg = W.MoEConfig("prequant", tokens, 1024, 512, 8, 3, seed=tokens, weights=weights,
+                      local_experts=4 if variant == "mask" else None)
+    wts = W.make_weights(cfg, device=cuda_device)
+    tw, ids = W.make_routing(cfg, device=cuda_device)
+    a1, a1s = A.per_group_quant_hip(W.make_hidden(cfg, device=cuda_device))
+    mask = W.make_expert_mask(cfg, device=cuda_device)
+    E = cfg.experts
+    n = torch.tensor([tokens - 9], dtype=torch.int32, device=cuda_device) \
+        if variant == "local_tokens" else None
+    dw = variant == "doweight"
+    dt = torch.float16 if variant == "fp16" else torch.bfloat16
+    out = W.run_layer(weights, a1, wts["w1"], wts["w2"], tw, ids, w1_scale=wts["w1_scale"],
+                      w2_scale=wts["w2_scale"], a1_scale=a1s, expert_mask=mask, dtype=dt,
+                      num_local_tokens=n, block_size_M=bm, doweight_stage1=dw)
+    bm = bm or A.default_block_m(tokens, 3, E, 1024, 512)
+    sid, sw, seid, nv, acc = A.moe_sorting(ids, tw, E, 1024, torch.float32, bm, mask, n)
+    st1, st2 = ((A.moe_stage1_a8w4, A.moe_stage2_a8w4) if weights == "mxfp4" else
+                (A.moe_stage1_fp8_blockscale, A.moe_stage2_fp8_blockscale))
+    a2, a2s = st1(a1, a1s, wts["w1"], wts["w1_scale"], sid, seid, nv, 3, bm, True,
+                  sorted_weights=sw if dw else None)
+    st2(a2, a2s, wts["w2"], wts["w2_scale"], sid, None if dw else sw, seid, nv, acc, bm, True)
+    rows = tokens - 9 if n is not None else tokens
+    ref, got = acc[:rows], out[:rows].float()
+    tol = ref.abs() * 2.0 ** (-10 if dt == torch.float16 else -8) + \
+        3 * 2.0 ** -23 * ref.abs().max() * 8
+    # stage 1 of the general and stream kernels may sum its K blocks from
+    # another start, which moves a few fp8 codes of a2 by a step
+    bad = ((got - ref).abs() > tol).float().mean().item()
+    assert bad <= (0.0 if bm >= 64 else 0.02), bad
+    _check(ref.cpu().numpy(), got.cpu().numpy(), "prequant")
+
+
+def test_prequant_layer_beyond_the_row_limit(cuda_device):
+    """The last token count on per-pair fp32 rows (1 GiB of them) and the first
+    on the fp32 accumulator give the same output for the tokens they share. Both
+    are rounded, so where their fp32 sums lie on two sides of a tie they differ
+    by a whole bf16 spacing, 2^-7 of the value at the foot of a binade; the
+    second term is the bound above."""
+    T, k, E, H, I = 8193, 8, 8, 4096, 128
+    cfg = W.MoEConfig("rows", T, H, I, E, k, seed=3)
+    wts = W.make_weights(cfg, device=cuda_device)
+    tw, ids = W.make_routing(cfg, device=cuda_device)
+    a1, a1s = A.per_group_quant_hip(W.make_hidden(cfg, device=cuda_device))
+    run = lambda n: W.run_layer("fp8", a1[:n], wts["w1"], wts["w2"], tw[:n], ids[:n],
+                                w1_scale=wts["w1_scale"], w2_scale=wts["w2_scale"],
+                                a1_scale=a1s[:n], block_size_M=64).float()
+    a, b = run(T)[:T - 1], run(T - 1)
+    assert ((a - b).abs() <= b.abs() * 2.0 ** -7 + 8 * 2.0 ** -23 * b.abs().max() * 8).all()
