@@ -19,9 +19,11 @@
 //   * the optional zero buffer (the fp32 accumulator of the down GEMM) is
 //     cleared for `tokens` rows, as the reference clears moe_buf.
 //
-// MI355X design (not the reference's LDS mesh + lane-group walk): tokens are
-// cut into chunks of `ct` tokens.  Each chunk builds an LDS bitmap
-// table[token][expert] of slot masks (a byte per cell for topk <= 8, a u32
+// MI355X design (not the reference's LDS mesh + lane-group walk): one workgroup
+// sorts a small batch; larger ones are cut into chunks of `ct` tokens, a
+// workgroup each. Up to 512 experts and 2048 pairs (of the batch or chunk) the
+// workgroup's LDS table holds one bit per (expert, pair) (the moe_sort_*bits
+// kernels below). Beyond, it is a bitmap table[token][expert] of slot masks (a byte per cell for topk <= 8, a u32
 // up to topk 32, so duplicates of an expert inside one token's top-k are all
 // kept, in slot order); a thread per expert then counts the expert's pairs
 // in each group of 8 rows (1 for u32 cells) into an LDS prefix, and a thread
@@ -94,10 +96,10 @@ __device__ __forceinline__ int sort_tokens(const SortParams& p) {
 
 // Clear the accumulator rows [0, tokens) and the whole second region with
 // 16-byte stores; run by the blocks of a launch that are not sorting.
-__device__ void zero_rows(const SortParams& p, int tokens, int block, int nblocks) {
+__device__ void zero_rows(const SortParams& p, int tokens, int block, int nblocks, int tid) {
     if (nblocks <= 0) return;
     const v4i z = {0, 0, 0, 0};
-    const int64_t first = (int64_t)block * kSortThreads + threadIdx.x;
+    const int64_t first = (int64_t)block * kSortThreads + tid;
     const int64_t stride = (int64_t)nblocks * kSortThreads;
     if (p.zero_buf) {
         const int64_t n16 = (int64_t)tokens * p.zero_row_bytes / 16;
@@ -108,6 +110,24 @@ __device__ void zero_rows(const SortParams& p, int tokens, int block, int nblock
         v4i* dst = reinterpret_cast<v4i*>(p.zero2);
         for (int64_t i = first; i < p.zero2_n16; i += stride) dst[i] = z;
     }
+}
+
+__device__ __forceinline__ void quant_side(const SortParams& p, int64_t block, int tid) {
+    if (p.q_bf16)
+        quant_groups_block<true>(p.qx, p.qq, p.qs, p.q_rows, p.q_cols, 0, p.q_num_rows, 1, block,
+                                 tid);
+    else
+        quant_groups_block<false>(p.qx, p.qq, p.qs, p.q_rows, p.q_cols, 0, p.q_num_rows, 1, block,
+                                  tid);
+}
+
+// The b-th 256 threads that do not sort: first the clearing blocks, then the
+// activation quant's.
+__device__ __forceinline__ void side_block(const SortParams& p, int tokens, int b, int tid) {
+    if (b < p.zero_blocks)
+        zero_rows(p, tokens, b, p.zero_blocks, tid);
+    else
+        quant_side(p, b - p.zero_blocks, tid);
 }
 
 // Clears the chunk counts once the scatter launch has read them, when they
@@ -381,15 +401,7 @@ __global__ __launch_bounds__(kSortThreads) void moe_sort_oneshot_kernel(SortPara
     extern __shared__ uint32_t smem[];
     const int tokens = sort_tokens(p);
     if ((int)blockIdx.x >= p.sort_blocks) {
-        const int b = (int)blockIdx.x - p.sort_blocks;
-        if (b < p.zero_blocks)
-            zero_rows(p, tokens, b, p.zero_blocks);
-        else if (p.q_bf16)
-            quant_groups_block<true>(p.qx, p.qq, p.qs, p.q_rows, p.q_cols, 0, p.q_num_rows, 1,
-                                     b - p.zero_blocks);
-        else
-            quant_groups_block<false>(p.qx, p.qq, p.qs, p.q_rows, p.q_cols, 0, p.q_num_rows, 1,
-                                      b - p.zero_blocks);
+        side_block(p, tokens, (int)blockIdx.x - p.sort_blocks, (int)threadIdx.x);
         return;
     }
     const SortLds L = carve_lds(p, smem);
@@ -403,21 +415,333 @@ __global__ __launch_bounds__(kSortThreads) void moe_sort_oneshot_kernel(SortPara
     scatter_pairs(p, L.table, 0, tokens, L.s_start, L.s_mask, L.s_pre);
 }
 
+// ---- a bit per pair: the one-workgroup sort, and a chunk's scatter ----
+// What sorting costs is latency: dependent memory round trips, barriers and
+// serial loops. So a thread loads its pairs' ids and weights once and keeps
+// them; the LDS table holds one bit per (expert, pair), in pair order, so that
+// a pair's rank is one prefix read and one population count; several lanes
+// share an expert's counting; one wave lays out the segments in registers; and
+// 16 or 64 lanes write an expert's padding side by side. Measured on MI355X
+// against the slot-mask tables, moe_sorting with the clearing of its buffer,
+// launches back to back in a graph: E = 256, top-8, one workgroup T=1 5.2 ->
+// 3.2 us, T=32 8.4 -> 4.2, T=128 16.4 -> 5.9, T=256 12.0 -> 7.9;
+// counts and scatter T=700 13.5 -> 10.0, T=2048 15.9 -> 11.4, T=8192 28.3 -> 20.0.
+constexpr int kBitPairs = 2048;       // of the batch, or of a chunk
+constexpr int kBitExperts = 512;
+constexpr size_t kBitLds = 112 * 1024;
+
+// u32 words of an expert's bits, odd so that consecutive experts' words sit in
+// different LDS banks
+__host__ __device__ inline int bit_pitch(int npairs) { return ((npairs + 31) / 32) | 1; }
+
+// Experts per lane of the layout scan: all of them over one wave.
+__host__ __device__ inline int bit_ept(int E) { return E <= 256 ? 4 : 8; }
+
+__host__ __device__ inline size_t bit_lds(int E, int npairs) {
+    return (size_t)64 * bit_ept(E) * 16 + (size_t)E * bit_pitch(npairs) * 6;
+}
+
+// Per expert (rounded up to whole lanes): its pairs (0 when masked off), those
+// in earlier chunks, its segment's start (-1 when masked off) and, with a
+// mask, its local id; then the bits and their per-word prefix.
+template <int EPT>
+struct BitLds {
+    int* cnt;
+    int* before;
+    int* start;
+    int* local;
+    uint32_t* bits;
+    uint16_t* pre;
+    int pitch;
+
+    __device__ __forceinline__ BitLds(uint32_t* smem, int E, int npairs) {
+        cnt = reinterpret_cast<int*>(smem);
+        before = cnt + 64 * EPT;
+        start = before + 64 * EPT;
+        local = start + 64 * EPT;
+        bits = reinterpret_cast<uint32_t*>(local + 64 * EPT);
+        pitch = bit_pitch(npairs);
+        pre = reinterpret_cast<uint16_t*>(bits + E * pitch);
+    }
+};
+
+// n / d by a float reciprocal: for n < 2^18, d <= 256 and a quotient below
+// 2^12, (n + 1/2) / d is at least 1/512 from an integer and its rounding error
+// below 2^-10, so it rounds to the right side
+__device__ __forceinline__ int div_small(int n, float rd) {
+    return (int)(((float)n + 0.5f) * rd);
+}
+
+// Inclusive sums over the wave in registers: shifts within the 16-lane rows,
+// then the row broadcasts.
+__device__ __forceinline__ int wave_scan_dpp(int v) {
+    v += __builtin_amdgcn_update_dpp(0, v, 0x111, 0xF, 0xF, false);
+    v += __builtin_amdgcn_update_dpp(0, v, 0x112, 0xF, 0xF, false);
+    v += __builtin_amdgcn_update_dpp(0, v, 0x114, 0xF, 0xF, false);
+    v += __builtin_amdgcn_update_dpp(0, v, 0x118, 0xF, 0xF, false);
+    v += __builtin_amdgcn_update_dpp(0, v, 0x142, 0xA, 0xF, false);
+    v += __builtin_amdgcn_update_dpp(0, v, 0x143, 0xC, 0xF, false);
+    return v;
+}
+
+// Clears the counts and bits; the mask waits in start / local for the layout
+// (experts past E have no pair). The caller's barrier publishes it.
+template <int NT, int EPT>
+__device__ __forceinline__ void bits_init(const SortParams& p, const BitLds<EPT>& L) {
+    const int E = p.E;
+    for (int e = threadIdx.x; e < 64 * EPT; e += NT) {
+        const int m = e >= E ? 0 : p.expert_mask ? p.expert_mask[e] : 1;
+        L.cnt[e] = 0;
+        L.before[e] = 0;
+        L.start[e] = m != 0 ? 0 : -1;
+        if (p.expert_mask) L.local[e] = m;
+    }
+    for (int i = threadIdx.x; i < E * L.pitch; i += NT) L.bits[i] = 0u;
+}
+
+template <int NT, int EPT, int PB>
+__device__ __forceinline__ void bits_set(const SortParams& p, const BitLds<EPT>& L,
+                                         const int (&pe)[PB]) {
+#pragma unroll
+    for (int u = 0; u < PB; ++u) {
+        const int i = u * NT + (int)threadIdx.x;
+        if (pe[u] >= 0 && pe[u] < p.E)
+            atomicOr(&L.bits[pe[u] * L.pitch + (i >> 5)], 1u << (i & 31));
+    }
+}
+
+// Per expert, the pairs before each word; with `total` the expert's count too.
+// Consecutive lanes share an expert, a run of words each.
+template <int NT, int EPT>
+__device__ __forceinline__ void bits_prefix(const SortParams& p, const BitLds<EPT>& L, int npairs,
+                                            bool total) {
+    const int E = p.E, tid = threadIdx.x;
+    const int nw = (npairs + 31) >> 5;
+    int tpe_log = 0;
+    while (tpe_log < 4 && (E << (tpe_log + 1)) <= NT) ++tpe_log;
+    const int tpe = 1 << tpe_log;
+    const int wpt = (nw + tpe - 1) >> tpe_log;
+    const int sub = tid & (tpe - 1);
+    const int w0 = min(sub * wpt, nw), w1 = min(w0 + wpt, nw);
+    for (int e0 = 0; e0 < E; e0 += NT >> tpe_log) {
+        const int e = e0 + (tid >> tpe_log);
+        const bool in = e < E;
+        const uint32_t* row = L.bits + (in ? e : 0) * L.pitch;
+        int cnt = 0;
+        for (int w = w0; w < w1; ++w) cnt += __popc(row[w]);
+        int incl = cnt;                                // over the expert's lanes
+        for (int o = 1; o < tpe; o <<= 1) {
+            const int n = __shfl_up(incl, o, 64);
+            if (sub >= o) incl += n;
+        }
+        if (in) {
+            int run = incl - cnt;
+            for (int w = w0; w < w1; ++w) {
+                L.pre[e * L.pitch + w] = (uint16_t)run;
+                run += __popc(row[w]);
+            }
+            if (total && sub == tpe - 1 && L.start[e] >= 0) L.cnt[e] = incl;
+        }
+    }
+}
+
+// n / bm of the segment layout: kSmall where the whole batch is kBitPairs pairs
+// (segment starts then lie below kBitPairs + kBitExperts * 256 < 2^18).
+template <bool kSmall>
+__device__ __forceinline__ int div_bm(int n, int bm, float rbm) {
+    return kSmall ? div_small(n, rbm) : n / bm;
+}
+
+// Segment layout from the counts, by the workgroup's first wave, EPT experts
+// per lane; `write`: num_valid_ids too.
+template <bool kSmall, int EPT>
+__device__ __forceinline__ void bits_layout(const SortParams& p, const BitLds<EPT>& L, int tokens,
+                                            bool write) {
+    if (threadIdx.x >= 64) return;
+    const int lane = threadIdx.x, bm = p.bm;
+    const float rbm = 1.0f / (float)bm;
+    int on[EPT], lo[EPT], nb[EPT], bsum = 0, msum = 0;
+#pragma unroll
+    for (int q = 0; q < EPT / 4; ++q) {
+        const v4i c = reinterpret_cast<const v4i*>(L.cnt)[lane * (EPT / 4) + q];
+        const v4i o = reinterpret_cast<const v4i*>(L.start)[lane * (EPT / 4) + q];
+        v4i l = {0, 0, 0, 0};
+        if (p.expert_mask) l = reinterpret_cast<const v4i*>(L.local)[lane * (EPT / 4) + q];
+#pragma unroll
+        for (int u = 0; u < 4; ++u) {
+            const int i = 4 * q + u;
+            on[i] = o[u];
+            lo[i] = l[u];
+            nb[i] = div_bm<kSmall>(c[u] + bm - 1, bm, rbm);
+            bsum += nb[i];
+            msum += lo[i];
+        }
+    }
+    const int bincl = wave_scan_dpp(bsum);
+    int bpre = bincl - bsum;
+    int mpre = p.expert_mask ? wave_scan_dpp(msum) - msum : 0;
+    if (write && lane == 63) {
+        p.num_valid[0] = bincl * bm;
+        p.num_valid[1] = tokens;
+    }
+#pragma unroll
+    for (int q = 0; q < EPT / 4; ++q) {
+        v4i st, l;
+#pragma unroll
+        for (int u = 0; u < 4; ++u) {
+            const int i = 4 * q + u;
+            st[u] = on[i] < 0 ? -1 : bpre * bm;
+            l[u] = mpre;
+            bpre += nb[i];
+            mpre += lo[i];
+        }
+        reinterpret_cast<v4i*>(L.start)[lane * (EPT / 4) + q] = st;
+        if (p.expert_mask) reinterpret_cast<v4i*>(L.local)[lane * (EPT / 4) + q] = l;
+    }
+}
+
+// The thread's pairs (of tokens t0 ..) to their places.
+template <int NT, int EPT, int PB>
+__device__ __forceinline__ void bits_emit(const SortParams& p, const BitLds<EPT>& L, int t0,
+                                          const int (&pe)[PB], const float (&pw)[PB]) {
+    const float rtk = 1.0f / (float)p.topk;
+#pragma unroll
+    for (int u = 0; u < PB; ++u) {
+        const int i = u * NT + (int)threadIdx.x, e = pe[u];
+        if (e < 0 || e >= p.E) continue;
+        const int start = L.start[e];
+        if (start < 0) continue;
+        const int t = div_small(i, rtk), w = e * L.pitch + (i >> 5);
+        const int pos = start + L.before[e] + L.pre[w] +
+                        __popc(L.bits[w] & ((1u << (i & 31)) - 1u));
+        p.sorted_ids[pos] =
+            (int32_t)(((uint32_t)(i - t * p.topk) << 24) | (uint32_t)(t0 + t));
+        p.sorted_w[pos] = pw[u];
+    }
+}
+
+// M-block ids and padding of experts first, first + step, ...: LPE lanes each.
+template <bool kSmall, int NT, int LPE, int EPT>
+__device__ __forceinline__ void bits_segments(const SortParams& p, const BitLds<EPT>& L,
+                                              int tokens, int first, int step) {
+    const int bm = p.bm, ln = threadIdx.x % LPE;
+    const float rbm = 1.0f / (float)bm;
+    const int32_t pad_id =
+        (int32_t)(((uint32_t)(p.topk & 0xFF) << 24) | ((uint32_t)tokens & 0xFFFFFFu));
+    for (int e = first + (int)threadIdx.x / LPE * step; e < p.E; e += NT / LPE * step) {
+        const int cnt = L.cnt[e];
+        if (cnt == 0) continue;
+        const int start = L.start[e];
+        const int nb = div_bm<kSmall>(cnt + bm - 1, bm, rbm), b0 = div_bm<kSmall>(start, bm, rbm);
+        const int eid = p.expert_mask ? L.local[e] : e;
+        for (int b = ln; b < nb; b += LPE) p.sorted_eids[b0 + b] = eid;
+        for (int i = start + cnt + ln; i < start + nb * bm; i += LPE) {
+            p.sorted_ids[i] = pad_id;
+            p.sorted_w[i] = 0.0f;
+        }
+    }
+}
+
+template <int NT, int EPT>
+__global__ __launch_bounds__(NT) void moe_sort_bits_kernel(SortParams p) {
+    extern __shared__ __attribute__((aligned(16))) uint32_t smem[];
+    const int tokens = sort_tokens(p);
+    if ((int)blockIdx.x >= p.sort_blocks) {
+        const int b = ((int)blockIdx.x - p.sort_blocks) * (NT / kSortThreads) +
+                      (int)threadIdx.x / kSortThreads;
+        if (b < p.zero_blocks + p.q_blocks) side_block(p, tokens, b, threadIdx.x % kSortThreads);
+        return;
+    }
+    constexpr int PB = kBitPairs / NT;                 // pairs per thread at most
+    const int npairs = tokens * p.topk;
+    const BitLds<EPT> L(smem, p.E, p.rows * p.topk);
+    int pe[PB];
+    float pw[PB];
+#pragma unroll
+    for (int u = 0; u < PB; ++u) {
+        const int i = u * NT + (int)threadIdx.x;
+        pe[u] = i < npairs ? p.topk_ids[i] : -1;
+        pw[u] = i < npairs ? p.topk_w[i] : 0.0f;
+    }
+    bits_init<NT>(p, L);
+    __syncthreads();
+    bits_set<NT>(p, L, pe);
+    __syncthreads();
+    bits_prefix<NT>(p, L, npairs, true);
+    __syncthreads();
+    bits_layout<true>(p, L, tokens, true);
+    __syncthreads();
+    bits_emit<NT>(p, L, 0, pe, pw);
+    bits_segments<true, NT, 16>(p, L, tokens, 0, 1);
+}
+
+// The scatter launch on the same table, a workgroup per chunk (see
+// moe_sort_scatter_kernel): the per-chunk counts are summed by all threads at
+// once, a slice of the chunks each, while the chunk's own pairs load.
+template <int NT, int EPT>
+__global__ __launch_bounds__(NT) void moe_sort_scatter_bits_kernel(SortParams p) {
+    extern __shared__ __attribute__((aligned(16))) uint32_t smem[];
+    if ((int)blockIdx.x >= p.num_chunks) {             // the activation quant, beside the chunks
+        const int b = ((int)blockIdx.x - p.num_chunks) * (NT / kSortThreads) +
+                      (int)threadIdx.x / kSortThreads + p.q_first;
+        if (b < p.q_blocks) quant_side(p, b, threadIdx.x % kSortThreads);
+        return;
+    }
+    constexpr int PB = kBitPairs / NT;
+    constexpr int kBatch = 16;                         // counts loaded per round trip
+    constexpr int kParts = NT / (64 * EPT);            // slices of the chunks
+    const int tokens = sort_tokens(p);
+    const int c = blockIdx.x, t0 = c * p.ct;
+    const int npairs = chunk_rows(p, c, tokens) * p.topk;
+    const BitLds<EPT> L(smem, p.E, p.ct * p.topk);
+    const int32_t* ids = p.topk_ids + (int64_t)t0 * p.topk;
+    const float* wts = p.topk_w + (int64_t)t0 * p.topk;
+    int pe[PB];
+    float pw[PB];
+#pragma unroll
+    for (int u = 0; u < PB; ++u) {
+        const int i = u * NT + (int)threadIdx.x;
+        pe[u] = i < npairs ? ids[i] : -1;
+        pw[u] = i < npairs ? wts[i] : 0.0f;
+    }
+    const int ce = threadIdx.x % (64 * EPT), part = threadIdx.x / (64 * EPT);
+    const int per = (p.num_chunks + kParts - 1) / kParts;
+    const int k1 = min((part + 1) * per, p.num_chunks);
+    int before = 0, total = 0;
+    if (ce < p.E)
+        for (int k = part * per; k < k1; k += kBatch) {
+            int v[kBatch];
+#pragma unroll
+            for (int u = 0; u < kBatch; ++u)
+                v[u] = k + u < k1 ? p.ws[(int64_t)(k + u) * p.E + ce] : 0;
+#pragma unroll
+            for (int u = 0; u < kBatch; ++u) {
+                before += k + u < c ? v[u] : 0;
+                total += v[u];
+            }
+        }
+    bits_init<NT>(p, L);
+    __syncthreads();
+    bits_set<NT>(p, L, pe);
+    if (ce < p.E && L.start[ce] >= 0) {
+        atomicAdd(&L.before[ce], before);
+        atomicAdd(&L.cnt[ce], total);
+    }
+    __syncthreads();
+    bits_layout<false>(p, L, tokens, c == 0);
+    bits_prefix<NT>(p, L, npairs, false);
+    __syncthreads();
+    bits_emit<NT>(p, L, t0, pe, pw);
+    bits_segments<false, NT, 64>(p, L, tokens, c, p.num_chunks);
+}
+
 // Per-chunk expert counts by an LDS histogram of the chunk's ids (every
 // (token, slot) pair with an id in range counts once, as in the table).
 __global__ __launch_bounds__(kSortThreads) void moe_sort_count_kernel(SortParams p) {
     extern __shared__ uint32_t smem[];
     const int tokens = sort_tokens(p);
     if ((int)blockIdx.x >= p.sort_blocks) {
-        const int b = (int)blockIdx.x - p.sort_blocks;
-        if (b < p.zero_blocks)
-            zero_rows(p, tokens, b, p.zero_blocks);
-        else if (p.q_bf16)
-            quant_groups_block<true>(p.qx, p.qq, p.qs, p.q_rows, p.q_cols, 0, p.q_num_rows, 1,
-                                     b - p.zero_blocks);
-        else
-            quant_groups_block<false>(p.qx, p.qq, p.qs, p.q_rows, p.q_cols, 0, p.q_num_rows, 1,
-                                      b - p.zero_blocks);
+        side_block(p, tokens, (int)blockIdx.x - p.sort_blocks, (int)threadIdx.x);
         return;
     }
     const int c = blockIdx.x;
@@ -452,11 +776,7 @@ constexpr int kChunkBatch = 16;   // per-chunk counts loaded per round trip
 __global__ __launch_bounds__(kSortThreads) void moe_sort_scatter_kernel(SortParams p) {
     extern __shared__ uint32_t smem[];
     if ((int)blockIdx.x >= p.num_chunks) {   // the activation quant, beside the chunks
-        const int b = (int)blockIdx.x - p.num_chunks + p.q_first;
-        if (p.q_bf16)
-            quant_groups_block<true>(p.qx, p.qq, p.qs, p.q_rows, p.q_cols, 0, p.q_num_rows, 1, b);
-        else
-            quant_groups_block<false>(p.qx, p.qq, p.qs, p.q_rows, p.q_cols, 0, p.q_num_rows, 1, b);
+        quant_side(p, (int)blockIdx.x - p.num_chunks + p.q_first, (int)threadIdx.x);
         return;
     }
     const int tokens = sort_tokens(p);
@@ -522,7 +842,15 @@ static int sort_chunk_tokens(int E, int topk, int64_t rows) {
     return ct;
 }
 
+// The one-workgroup sort: few enough pairs, and an LDS table that fits. A
+// forced chunk size (AITER_AMD_SORT_CT) means the chunked kernels.
+static bool sort_in_bits(int64_t rows, int64_t topk, int64_t E) {
+    return rows * topk <= kBitPairs && E <= kBitExperts &&
+           bit_lds((int)E, (int)(rows * topk)) <= kBitLds && !getenv("AITER_AMD_SORT_CT");
+}
+
 int64_t sort_workspace_bytes(int64_t rows, int64_t topk, int64_t E) {
+    if (sort_in_bits(rows, topk, E)) return 0;
     int ct = sort_chunk_tokens((int)E, (int)topk, rows);
     int64_t chunks = ceil_div(rows > 0 ? rows : 1, ct);
     if (chunks <= 1) return 0;
@@ -598,7 +926,21 @@ bool launch_moe_sort(const int32_t* topk_ids, const float* topk_w, const int32_t
         p.q_blocks = (int)qb;
         quant_done = true;
     }
-    if (p.num_chunks == 1) {
+    if (sort_in_bits(rows, topk, E)) {
+        p.sort_blocks = 1;
+        const size_t lds = bit_lds((int)E, (int)(rows * topk));
+        const int64_t side = zero_blocks + p.q_blocks;
+        auto go = [&](auto kern, int nt) {
+            hipLaunchKernelGGL(kern, dim3(1 + (unsigned)ceil_div(side, nt / kSortThreads)), dim3(nt),
+                               lds, stream, p);
+        };
+        if (E > 256)
+            go(moe_sort_bits_kernel<1024, 8>, 1024);
+        else if (rows * topk <= 256 && E <= 64)
+            go(moe_sort_bits_kernel<256, 4>, 256);
+        else
+            go(moe_sort_bits_kernel<1024, 4>, 1024);
+    } else if (p.num_chunks == 1) {
         p.sort_blocks = 1;
         hipLaunchKernelGGL(moe_sort_oneshot_kernel, dim3(1 + zero_blocks + p.q_blocks),
                            dim3(kSortThreads), full_lds, stream, p);
@@ -629,9 +971,22 @@ bool launch_moe_sort(const int32_t* topk_ids, const float* topk_w, const int32_t
         hipLaunchKernelGGL(moe_sort_count_kernel,
                            dim3(p.num_chunks + zero_blocks + q_count),
                            dim3(kSortThreads), (size_t)E * 4, stream, p);
-        hipLaunchKernelGGL(moe_sort_scatter_kernel,
-                           dim3(p.num_chunks + (p.q_blocks - q_count)),
-                           dim3(kSortThreads), full_lds, stream, p);
+        const int64_t cpairs = (int64_t)p.ct * topk;
+        if (cpairs <= kBitPairs && E <= kBitExperts && bit_lds((int)E, (int)cpairs) <= kBitLds) {
+            const dim3 grid(p.num_chunks +
+                            (unsigned)ceil_div(p.q_blocks - q_count, 1024 / kSortThreads));
+            const size_t lds = bit_lds((int)E, (int)cpairs);
+            if (E <= 256)
+                hipLaunchKernelGGL((moe_sort_scatter_bits_kernel<1024, 4>), grid, dim3(1024), lds,
+                                   stream, p);
+            else
+                hipLaunchKernelGGL((moe_sort_scatter_bits_kernel<1024, 8>), grid, dim3(1024), lds,
+                                   stream, p);
+        } else {
+            hipLaunchKernelGGL(moe_sort_scatter_kernel,
+                               dim3(p.num_chunks + (p.q_blocks - q_count)),
+                               dim3(kSortThreads), full_lds, stream, p);
+        }
         if (ws_in_buf) {
             const int64_t nb = std::min<int64_t>(ceil_div(p.zero_skip16, kSortThreads), 1024);
             hipLaunchKernelGGL(moe_sort_clear_kernel, dim3(nb), dim3(kSortThreads), 0, stream,

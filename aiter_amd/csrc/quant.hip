@@ -28,7 +28,7 @@ __global__ __launch_bounds__(kQuantThreads) void per_group_quant_fp8_kernel(
     int64_t rows, int cols, int transpose_scale, const int32_t* __restrict__ num_rows,
     int num_rows_factor) {
     quant_groups_block<kBf16>(x, q, scale, rows, cols, transpose_scale, num_rows,
-                              num_rows_factor, (int64_t)blockIdx.x);
+                              num_rows_factor, (int64_t)blockIdx.x, (int)threadIdx.x);
 }
 
 void launch_per_group_quant_fp8(const void* x, int x_dtype, void* q, float* scale, int64_t rows,

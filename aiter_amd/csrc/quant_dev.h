@@ -1,6 +1,6 @@
 // 1 x 128 FP8 quantisation of one 256-thread block's 16 groups: the body of
 // per_group_quant_fp8_kernel, shared with the sorting launch (which runs it
-// in extra blocks at decode sizes). Semantics: quant.hip's header.
+// in extra blocks at decode sizes; `tid` is the thread within the 256). Semantics: quant.hip's header.
 #pragma once
 #include "common.h"
 
@@ -49,15 +49,15 @@ __device__ __forceinline__ void quant_groups_block(const uint16_t* __restrict__ 
                                                    float* __restrict__ scale, int64_t rows,
                                                    int cols, int transpose_scale,
                                                    const int32_t* __restrict__ num_rows,
-                                                   int num_rows_factor, int64_t block) {
+                                                   int num_rows_factor, int64_t block, int tid) {
     int64_t rows_eff = rows;
     if (num_rows) {
         int64_t r = (int64_t)num_rows[0] * num_rows_factor;
         rows_eff = r < 0 ? 0 : (r < rows ? r : rows);
     }
     const int G = cols / 128;
-    const int64_t g = block * (kQuantThreads / 16) + (threadIdx.x >> 4);
-    const int sub = threadIdx.x & 15;
+    const int64_t g = block * (kQuantThreads / 16) + (tid >> 4);
+    const int sub = tid & 15;
     const int64_t row = g / G;
     const int gc = (int)(g - row * G);
     const bool active = row < rows_eff;

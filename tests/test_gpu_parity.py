@@ -94,6 +94,36 @@ def test_sorting_chunk_size_invariant(cuda_device, monkeypatch, ct):
     assert torch.count_nonzero(buf).item() == 0
 
 
+# both sides of every limit of the one-bit-per-pair sort: words of 32 pairs,
+# 2048 pairs in one workgroup, 256 and 512 experts, its LDS table, one thread's
+# second pair; block sizes that divide by 1 and by the largest; chunks of the
+# scatter launch with a last partial one
+@pytest.mark.parametrize("T,E,k,bm,masked,local", [
+    (1, 1, 1, 1, False, None), (31, 7, 1, 16, True, None), (32, 64, 1, 1, False, None),
+    (33, 65, 1, 256, True, None), (128, 64, 2, 32, True, 0), (129, 64, 2, 32, False, 77),
+    (256, 256, 8, 16, True, 255), (257, 256, 8, 1, False, None), (227, 257, 9, 256, True, None),
+    (228, 257, 9, 48, False, 200), (64, 512, 8, 16, True, None), (200, 512, 8, 16, False, None),
+    (64, 513, 8, 16, True, None), (64, 40, 32, 16, False, None), (65, 40, 32, 16, True, 40),
+    (700, 512, 8, 64, True, None), (701, 256, 8, 256, False, 650), (5000, 300, 8, 1, True, 4999),
+    (700, 513, 8, 64, False, None)])
+def test_sorting_bit_table_edges(cuda_device, T, E, k, bm, masked, local):
+    ids, w = _routing_np(T, E, k, seed=T * 3 + E)
+    if k > 1:
+        ids[T // 2, 1] = ids[T // 2, 0]       # a duplicate inside one token's top-k
+    ids[T - 1, k - 1] = E                     # out of range
+    mask = np.random.default_rng(E).integers(0, 2, E).astype(np.int32) if masked else None
+    dev = lambda a, dt=None: None if a is None else torch.as_tensor(a, dtype=dt, device=cuda_device)
+    loc = dev([local], torch.int32) if local is not None else None
+    sid, sw, se, nv, buf = A.moe_sorting(dev(ids), dev(w), E, 256, torch.bfloat16, bm, dev(mask), loc)
+    ref = R.moe_sorting_argsort(ids, w, E, bm, mask, local)
+    assert torch.count_nonzero(buf[:T if local is None else local]).item() == 0
+    assert np.array_equal(_np(nv), ref[3])
+    n = int(ref[3][0])
+    assert np.array_equal(_np(sid)[:n], ref[0])
+    assert np.array_equal(_np(sw)[:n].view(np.int32), ref[1].view(np.int32))
+    assert np.array_equal(_np(se)[: n // bm], ref[2])
+
+
 def test_sorting_worked_example(cuda_device):
     """The reference's worked example (csrc/include/moe_sorting_opus.h:277-339,
     fixture tests/golden/moe_sorting_worked_example.json), every output array."""
