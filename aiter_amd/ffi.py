@@ -9,8 +9,8 @@ name the way the reference's `compile_ops(..., ffi_type="ctypes")` does
     bool -> int,  float -> float,  str / Optional[str] -> const char*
     (appended)                -> hipStream_t: torch's current stream
 
-A call clears the library's last error, calls, and raises RuntimeError with
-`aiter_get_last_error()` when the status is non-zero or an error was left.
+A call raises RuntimeError with `aiter_get_last_error()` when the status is
+non-zero (each entry clears the last error first).
 The stubs below carry the reference's names and signatures
 (aiter/ops/moe_sorting.py:11-25, aiter/ops/quant.py:472-481,
 aiter/ops/moe_op.py:15-42, 172-213, 295-340, aiter/ops/activation.py:10-19,
@@ -213,10 +213,11 @@ def ctypes_op(func):
                 _pack_desc(raw, off, v, dev)
                 cargs.append(base + off)
                 off += _DESC.size
-        lib.aiter_clear_last_error()
+        # the entry clears the last error itself and leaves one only with a
+        # non-zero status (safe_call)
         rc = fn(*cargs, None if device is None else _stream_of(device))
-        err = lib.aiter_get_last_error()
-        if rc != 0 or err:
+        if rc != 0:
+            err = lib.aiter_get_last_error()
             lib.aiter_clear_last_error()
             raise RuntimeError(f"{func.__name__} failed: "
                                f"{err.decode(errors='replace') if err else f'status {rc}'}")

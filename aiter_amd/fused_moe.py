@@ -26,7 +26,7 @@ from . import _abi, ffi
 from .enums import AITER_DTYPE, ActivationType, QuantType, dtypes, quant_remap
 from .quant import e8m0_unshuffle, per_group_quant_hip
 from .topk import fused_topk  # noqa: F401  (aiter.fused_moe.fused_topk)
-from .tune import tuned_block_m, tuned_config
+from .tune import _CLEAR_WITH, tuned_block_m, tuned_config
 
 BLOCK_SIZE_M = 32
 
@@ -40,6 +40,49 @@ def _stream(dev: torch.device) -> int:
     if _RAW_STREAM is not None and dev.index is not None:
         return _RAW_STREAM(dev.index)
     return torch.cuda.current_stream(dev).cuda_stream
+
+
+# The switches that a layer call reads (AITER_AMD_*), from os.environ's own
+# table where it is there: os.environ.get of a name that is not set encodes it
+# and raises and catches a KeyError, about 1 us, and a call reads five. Both
+# see changes at once.
+_ENV_TABLE = getattr(os.environ, "_data", None)
+if not isinstance(_ENV_TABLE, dict) or (_ENV_TABLE and
+                                        not isinstance(next(iter(_ENV_TABLE)), bytes)):
+    _ENV_TABLE = None
+_SWITCHES = ("AITER_AMD_TUNED_FMOE", "AITER_AMD_FUSED", "AITER_AMD_ST_KSPLIT1",
+             "AITER_AMD_SORT_CT")
+_SWITCH_KEYS = tuple(n.encode() for n in _SWITCHES)
+
+
+def _switches() -> tuple:
+    """The values of _SWITCHES (None: not set), part of the cached plans' key."""
+    if _ENV_TABLE is None:
+        return tuple(os.environ.get(n) for n in _SWITCHES)
+    get = _ENV_TABLE.get
+    a, b, c, d = _SWITCH_KEYS
+    return get(a), get(b), get(c), get(d)
+
+
+@functools.lru_cache(maxsize=4096)
+def _layer_plan(M, model_dim, inter_dim, E, global_E, topk, block_size_M, a8w4, prequant, device,
+                switches):
+    """(block_m, one-launch layer, workspace bytes) of a layer call: the table and
+    heuristic lookups below and the library's workspace query, kept per shape
+    and switch values."""
+    if block_size_M not in (None, -1):
+        block_m = int(block_size_M)
+    else:
+        block_m = select_block_m(M, topk, E, model_dim, inter_dim, a8w4, device, global_E)
+    if prequant:
+        return block_m, False, _layer_workspace_bytes(
+            M, model_dim, inter_dim, E, global_E, topk, block_m,
+            "aiter_amd_fused_moe_prequant_workspace_bytes")
+    one = select_run_1stage(M, topk, E, model_dim, inter_dim, a8w4, block_m, device)
+    return block_m, one, _layer_workspace_bytes(M, model_dim, inter_dim, E, global_E, topk, block_m)
+
+
+_CLEAR_WITH.append(_layer_plan.cache_clear)
 
 
 def _layer_workspace_bytes(M: int, model_dim: int, inter_dim: int, E: int, global_E: int,
@@ -177,12 +220,18 @@ def fused_moe(
     """Same signature and result as aiter.fused_moe.fused_moe (fused_moe.py:118-169);
     runs the registered custom op torch.ops.aiter_amd.fused_moe_ as the reference
     runs torch.ops.aiter.fused_moe_ (fused_moe.py:172-205)."""
-    return torch.ops.aiter_amd.fused_moe_(
+    return _layer_op()(
         hidden_states, w1, w2, topk_weight, topk_ids, expert_mask, int(activation),
         int(quant_type), bool(doweight_stage1), w1_scale, w2_scale, a1_scale, a2_scale,
         int(block_size_M) if block_size_M else -1, num_local_tokens,
         int(moe_sorting_dispatch_policy), dtype, int(hidden_pad), int(intermediate_pad), bias1,
         bias2)
+
+
+@functools.lru_cache(maxsize=1)
+def _layer_op():
+    # the overload itself: the packet would resolve it on every call
+    return torch.ops.aiter_amd.fused_moe_.default
 
 
 def fused_moe_a8w4(
@@ -430,7 +479,8 @@ def _fused_moe_impl(hidden_states, w1, w2, topk_weight, topk_ids, expert_mask, a
                     block_size_M, num_local_tokens, moe_sorting_dispatch_policy, dtype,
                     hidden_pad, intermediate_pad, bias1, bias2, a8w4):
     activation = ActivationType(activation)
-    quant_type = quant_remap.get(QuantType(quant_type), QuantType(quant_type))
+    quant_type = QuantType(quant_type)
+    quant_type = quant_remap.get(quant_type, quant_type)
     M, topk = topk_ids.shape
     E, model_dim, inter_dim = get_inter_dim(tuple(w1.shape), tuple(w2.shape))
     if w1.shape[1] != 2 * inter_dim:
@@ -448,12 +498,8 @@ def _fused_moe_impl(hidden_states, w1, w2, topk_weight, topk_ids, expert_mask, a
     if bool(getattr(w2, "is_shuffled", False)) != shuffled:
         raise ValueError("w1 and w2 must both be shuffled or both be plain")
     global_E = expert_mask.numel() if expert_mask is not None else E
-    if block_size_M not in (None, -1):
-        block_m = int(block_size_M)
-    else:
-        block_m = select_block_m(M, topk, E, model_dim, inter_dim, a8w4, topk_ids.device,
-                                 global_E)
     device = topk_ids.device
+    prequant = hidden_states.dtype == dtypes.fp8
     topk_ids = topk_ids.to(torch.int32).contiguous()
     topk_weight = topk_weight.to(torch.float32).contiguous()
     w1c, w2c = w1.contiguous(), w2.contiguous()
@@ -466,13 +512,13 @@ def _fused_moe_impl(hidden_states, w1, w2, topk_weight, topk_ids, expert_mask, a
     if M == 0:
         return out
     stream = _stream(device)
+    block_m, one, ws_bytes = _layer_plan(M, model_dim, inter_dim, E, global_E, topk, block_size_M,
+                                         a8w4, prequant, device, _switches())
+    ws = torch.empty(ws_bytes, dtype=torch.uint8, device=device)
 
-    if hidden_states.dtype != dtypes.fp8:
+    if not prequant:
         # one C-ABI call runs the whole layer
         x = hidden_states.contiguous()
-        ws_bytes = _layer_workspace_bytes(M, model_dim, inter_dim, E, global_E, topk, block_m)
-        ws = torch.empty(ws_bytes, dtype=torch.uint8, device=device)
-        one = select_run_1stage(M, topk, E, model_dim, inter_dim, a8w4, block_m, device)
         _abi.call(
             ("aiter_amd_fused_moe_1stage_a8w4" if one else "aiter_amd_fused_moe_a8w4") if a8w4
             else ("aiter_amd_fused_moe_1stage_fp8_blockscale" if one
@@ -487,9 +533,6 @@ def _fused_moe_impl(hidden_states, w1, w2, topk_weight, topk_ids, expert_mask, a
     # fp8 activations with caller-provided 1x128 scales: no quant step, and a
     # token's weighted rows are summed in fp32
     a1, a1s = hidden_states.contiguous(), a1_scale.contiguous()
-    ws_bytes = _layer_workspace_bytes(M, model_dim, inter_dim, E, global_E, topk, block_m,
-                                      "aiter_amd_fused_moe_prequant_workspace_bytes")
-    ws = torch.empty(ws_bytes, dtype=torch.uint8, device=device)
     s1, s2 = w1s.data_ptr(), w2s.data_ptr()
     _abi.call(
         "aiter_amd_fused_moe_prequant", a1.data_ptr(), a1s.data_ptr(), w1c.data_ptr(),

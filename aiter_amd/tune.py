@@ -73,10 +73,16 @@ def tuned_config(cu_num: int, token: int, model_dim: int, inter_dim: int, expert
                    padded_tokens(token), model_dim, inter_dim, expert, topk, q_type, q_dtype_w)
 
 
+# further caches of what the tables say (a layer's plan), cleared with them
+_CLEAR_WITH: list = []
+
+
 def clear_cache() -> None:
     """Forget the loaded tables and their lookups (after a table file changed)."""
     _load.cache_clear()
     _config.cache_clear()
+    for clear in _CLEAR_WITH:
+        clear()
 
 
 @functools.lru_cache(maxsize=4096)
