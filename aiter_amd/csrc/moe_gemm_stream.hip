@@ -24,10 +24,12 @@
 // The K loop is unrolled by D with D operand buffers: step k computes from
 // buffer k % D and then refills it with step k + D, so D steps of loads are
 // always outstanding and the compiler's wait counts target the oldest.
-// Weight loads are non-temporal: each weight byte is used by one workgroup
-// once, so it should not displace the activations and scales in the caches.
+// Weights that one M-block alone reads are loaded non-temporally (each byte is
+// used once and should displace nothing); the M-blocks of an expert with
+// several walk its weights in step, through ordinary loads, in one L2.
 #include <algorithm>
 #include <cstdlib>
+#include <type_traits>
 
 #include "common.h"
 #include "quant_dev.h"
@@ -65,7 +67,7 @@ struct Args {
     int topk;
     int E;
     int64_t a_rows;
-    int ntw;                   // stage 2: 256-column groups per workgroup, one K loop
+    int ntw;                   // stage 2: 256-column groups per workgroup (0: walk_groups)
     // stage 1 split-K: ksplit workgroups per tile, each over KB / ksplit K
     // steps, leave fp32 partial sums in kpart; the last to arrive (counted in
     // kcnt[tile], zero on entry and left zero) adds them in split order and
@@ -97,6 +99,7 @@ struct Args {
     // sorted_eids holds one expert per BM << eid_shift sorted rows: a caller's
     // 64- or 128-row M-blocks are walked as 32-row ones
     int eid_shift;
+    int gx;                    // stage 1: column tiles x ksplit; stage 2: 256-column groups
     // direct M-blocks, for a layer too small to be worth a sorting launch:
     // with dir_ids set, M-block p holds routing pair p = token * topk + slot
     // of dir_tokens tokens in its first row (the rest is padding), its expert
@@ -112,6 +115,52 @@ struct Args {
     int xq_bf16;
 };
 
+// Workgroup L (x fastest) of the grid -> (column tile, M-block), L on XCD L % 8. Where 8
+// divides the gx column tiles, column by column: XCD x then runs tiles x, x + 8,
+// ... of every M-block, and M-blocks of one expert meet its weights in one L2.
+// Otherwise XCD x takes groups of four consecutive M-blocks (the groups x, x +
+// 8, ...) through all their column tiles, the M-blocks of a group side by side,
+// and the last mv % 32 of the mv valid M-blocks go column by column, so that
+// every XCD gets as many workgroups. Measured on MI355X against column by
+// column throughout (with shared weights loaded as below), skewed routing at
+// 32-row blocks: hidden 3072, inter 768, T=256 152 -> 143 us, hidden 4096,
+// inter 384, 128 experts, T=500 186 -> 171 us; uniform routing level.
+__device__ __forceinline__ void tile_of(int L, int gx, int mv, int& bx, int& mb) {
+    const int full = (gx & 7) != 0 ? mv & ~31 : 0;
+    if (L < full * gx) {
+        const int per = gx * 4, idx = L >> 3;
+        const int grp = idx / per, r = idx - grp * per;
+        bx = r >> 2;
+        mb = (grp * 8 + (L & 7)) * 4 + (r & 3);
+    } else {
+        const int q = L - full * gx, m = q / gx;
+        bx = q - m * gx;
+        mb = full + m;
+    }
+}
+
+// Stage 2's 256-column groups per workgroup, from the M-blocks that routing
+// gave (the host knows only how many there could be). A workgroup streams 256 x
+// K weight bytes per group, so its setup and epilogue weigh more the fewer
+// groups it walks; but the walk has to leave most CUs a workgroup, and the last
+// of the ~512 that run at a time should not be nearly empty. Measured on MI355X
+// (layer, us, at one / two / four groups; mv M-blocks): fp8, 16 K steps, 16
+// groups: mv 101 431 / 424 / 420, mv 160 678 / 666 / 666, mv 219 873 / 848 /
+// 874; 3 steps: mv 122 112 / 110 / 111; 6 steps, 12 groups: mv 101 127 / 132 /
+// 136, mv 250 281 / 280 / 280; 2 steps, 28 groups: mv 18 45.9 / 43.4 / 44.5, mv
+// 250 248 / 238 / 235. MXFP4, 16 steps: mv 160 363 / 370 / 354, mv 250 528 /
+// 540 / 517, skewed routing at T=64 142 / 147 / 163.
+template <bool W4>
+__device__ __forceinline__ int walk_groups(int mv, int groups, int KB) {
+    const bool two = (groups & 1) == 0 && 2 * KB <= kMaxKB;
+    const bool four = (groups & 3) == 0 && 4 * KB <= kMaxKB;
+    const int w2 = mv * groups / 2, w4 = w2 / 2;           // workgroups
+    if (KB <= 2) return four && w4 >= 256 ? 4 : two ? 2 : 1;
+    if (W4) return four && w4 >= 600 ? 4 : 1;
+    if (four && KB >= 8 && w4 >= 384 && w4 <= 512) return 4;
+    return two && (w2 >= 3 * 512 || (w2 >= 384 && (w2 & 511) >= 256)) ? 2 : 1;
+}
+
 // One K step of one wave's operands.
 template <int NRT, bool W4>
 struct Step {
@@ -122,7 +171,8 @@ struct Step {
 // STAGE 1: gate+up GEMM -> SiLU*up -> a2 (fp8 + 1x128 scales); STAGE 2:
 // down GEMM accumulated into acc; STAGE 3: both for one 128-wide slice of
 // the intermediate dim per workgroup (the fused layer).
-template <int BM, int STAGE, bool SHUFFLED, bool W4, int D, bool XQ = false>
+// ACC32: stage 2 adds into an fp32 accumulator (else bf16 / fp16, acc_dtype).
+template <int BM, int STAGE, bool SHUFFLED, bool W4, int D, bool XQ = false, bool ACC32 = true>
 __global__ __launch_bounds__(kThreads) void moe_gemm_stream_kernel(Args g) {
     constexpr int NRT = BM / 16;
     constexpr bool G1 = STAGE != 2;                      // runs the gate+up GEMM
@@ -152,20 +202,35 @@ __global__ __launch_bounds__(kThreads) void moe_gemm_stream_kernel(Args g) {
     const int lr = lane & 15;
     const int lq = lane >> 4;
 
-    const int mb = blockIdx.y;
     const bool direct = g.dir_ids != nullptr;
     const int nvalid = direct ? g.dir_tokens * g.topk * BM : g.num_valid[0];
-    if (mb * BM >= nvalid) return;
+    // (column tile x K range, M-block) of the workgroup; stage 2 walks ntw
+    // consecutive 256-column groups in one K loop (steps s = jt * KB + kb)
+    const int mv = (nvalid + BM - 1) / BM;
+    const int ntw = STAGE != 2 ? 1 : g.ntw > 0 ? g.ntw : walk_groups<W4>(mv, g.gx, g.K / 128);
+    int bx = blockIdx.x, mb = blockIdx.y;
+    if (ntw > 1 || ((g.gx & 7) != 0 && mv >= 32))
+        tile_of((int)(blockIdx.y * gridDim.x + blockIdx.x), g.gx / ntw, mv, bx, mb);
+    if (mb >= mv) return;
     const int tokens = direct ? g.dir_tokens : g.num_valid[1];
-    const int e = direct ? g.dir_ids[mb] : g.sorted_eids[mb >> g.eid_shift];
+    // Whether another M-block of this expert (they are neighbours) reads the
+    // same weights; the three ids load together
+    int e, ep = -1, en = -1;
+    if (direct) {
+        e = g.dir_ids[mb];
+    } else {
+        e = g.sorted_eids[mb >> g.eid_shift];
+        if constexpr (!FUSED) {
+            ep = g.sorted_eids[max(mb - 1, 0) >> g.eid_shift];
+            en = g.sorted_eids[min(mb + 1, mv - 1) >> g.eid_shift];
+        }
+    }
+    const bool shared_w = (ep == e && mb > 0) || (en == e && mb + 1 < mv);
     if (e < 0 || e >= g.E) return;
-    // stage 2 may walk ntw consecutive 256-column groups in one K loop (steps
-    // s = jt * KB + kb); stage 1 always has one tile, whose K range the S
-    // workgroups blockIdx.x = tile * S + ks split
-    const int ntw = STAGE == 2 ? g.ntw : 1;
+    // stage 1's tile has its K range split by S workgroups bx = tile * S + ks
     const int S = G1 ? g.ksplit : 1;
-    const int nt = (int)blockIdx.x / S;
-    const int ks = (int)blockIdx.x - nt * S;
+    const int nt = bx / S;
+    const int ks = bx - nt * S;
     if (S > 1 && mb >= g.kmb) return;    // never: a routed M-block holds >= 1 of the tokens*topk pairs
     const int n0 = nt * (G1 ? 128 : 256 * ntw);
 
@@ -253,24 +318,33 @@ __global__ __launch_bounds__(kThreads) void moe_gemm_stream_kernel(Args g) {
     __syncthreads();
 
     // ---- per-lane operand sources (K step 0) ----
+    // The tile's weight rows as buffer resources (stage 1: 128 gate rows and
+    // the matching 128 up rows; stage 2: the 256 * ntw output columns), read
+    // at a 32-bit lane offset plus a wave-uniform step offset: no 64-bit lane
+    // address per column tile and step in flight.
     const uint8_t* we = g.w + (int64_t)e * g.N * KBY;
-    const uint8_t* bsrc[kNCT];
+    const int rbytes = (G1 ? 128 : 256 * ntw) * KBY;
+    __amdgpu_buffer_rsrc_t rb[2];
+#pragma unroll
+    for (int h = 0; h < 2; ++h)
+        rb[h] = __builtin_amdgcn_make_buffer_rsrc(
+            const_cast<uint8_t*>(we + (int64_t)(n0 + (G1 && h ? g.inter : 0)) * KBY), (short)0,
+            rbytes, 0x00020000);
+    uint32_t boff[kNCT];
     const uint8_t* bssrc[kNCT];
 #pragma unroll
     for (int ct = 0; ct < kNCT; ++ct) {
-        int row0;
-        if (G1)
-            row0 = ct < 2 ? n0 + 32 * wv + 16 * ct : g.inter + n0 + 32 * wv + 16 * (ct - 2);
-        else
-            row0 = n0 + 64 * wv + 16 * ct;
+        // first row of the 16-row group, in its resource
+        const int row0 = G1 ? 32 * wv + 16 * (ct & 1) : 64 * wv + 16 * ct;
         if (W4)
-            bsrc[ct] = SHUFFLED ? we + (int64_t)row0 * KBY + lane * 16
-                                : we + (int64_t)(row0 + lr) * KBY + lq * 16;
+            boff[ct] = SHUFFLED ? (uint32_t)(row0 * KBY + lane * 16)
+                                : (uint32_t)((row0 + lr) * KBY + lq * 16);
         else
-            bsrc[ct] = SHUFFLED ? we + (int64_t)row0 * K + lq * 512 + lr * 16
-                                : we + (int64_t)(row0 + lr) * K + lq * 32;
+            boff[ct] = SHUFFLED ? (uint32_t)(row0 * K + lq * 512 + lr * 16)
+                                : (uint32_t)((row0 + lr) * K + lq * 32);
         // A8W4: the e8m0 bytes of the lane's weight row (all four lane quarters)
-        bssrc[ct] = W4 ? g.w_scale8 + ((int64_t)e * g.N + row0 + lr) * (K / 32) : nullptr;
+        const int wrow = n0 + (G1 && ct >= 2 ? g.inter : 0) + row0 + lr;
+        bssrc[ct] = W4 ? g.w_scale8 + ((int64_t)e * g.N + wrow) * (K / 32) : nullptr;
     }
     constexpr int BSTEP = W4 ? (SHUFFLED ? 1024 : 64) : (SHUFFLED ? 2048 : 128);
     constexpr int BHI = SHUFFLED ? 256 : 16;       // fp8: offset of the fragment's second half
@@ -282,27 +356,6 @@ __global__ __launch_bounds__(kThreads) void moe_gemm_stream_kernel(Args g) {
         if (arow < 0) arow = 0;                    // pad rows: any valid row, result unused
         asrc[rt] = g.a + (int64_t)arow * K + (W4 ? lq * 16 : lq * 32);
     }
-
-    // operands of K block kb of column group jt
-    auto load = [&](Step<NRT, W4>& s, int kb, int jt) {
-#pragma unroll
-        for (int ct = 0; ct < kNCT; ++ct) {
-            const uint8_t* p = bsrc[ct] + (int64_t)kb * BSTEP + (int64_t)jt * 256 * KBY;
-            s.b[ct][0] = __builtin_nontemporal_load(reinterpret_cast<const v4i*>(p));
-            if (!W4)
-                s.b[ct][W4 ? 0 : 1] =
-                    __builtin_nontemporal_load(reinterpret_cast<const v4i*>(p + BHI));
-        }
-        // XQ: A comes from LDS when the step is computed (no registers held)
-        if constexpr (!XQ) {
-#pragma unroll
-            for (int rt = 0; rt < NRT; ++rt) {
-                const uint8_t* p = asrc[rt] + kb * 128;
-                s.a[rt][0] = *reinterpret_cast<const v4i*>(p);
-                s.a[rt][1] = *reinterpret_cast<const v4i*>(p + AHI);
-            }
-        }
-    };
 
     v4f acc[NRT][kNCT];
 #pragma unroll
@@ -329,7 +382,8 @@ __global__ __launch_bounds__(kThreads) void moe_gemm_stream_kernel(Args g) {
                 const v2i v = *reinterpret_cast<const v2i*>(p);
                 dst[ct][0] = v[0], dst[ct][1] = v[1];
             } else {
-                dst[ct][0] = *reinterpret_cast<const int*>(p);
+#pragma unroll
+                for (int d = 0; d < D; ++d) dst[ct][d] = reinterpret_cast<const int*>(p)[d];
             }
         }
     };
@@ -374,27 +428,71 @@ __global__ __launch_bounds__(kThreads) void moe_gemm_stream_kernel(Args g) {
         }
     };
 
-    // ---- stage 2 epilogue of column group jt: weighted fp32 atomics ----
-    auto epilogue2 = [&](int jt) {
+    // ---- stage 2 epilogue of column group jt: weighted atomics. One branch on
+    // the accumulator's type: the few steps of a short K range are bound by the
+    // code they fetch ----
+    auto epilogue2 = [&](int jt) __attribute__((always_inline)) {
+        auto rows = [&](auto add) __attribute__((always_inline)) {
 #pragma unroll
-        for (int rt = 0; rt < NRT; ++rt)
+            for (int rt = 0; rt < NRT; ++rt)
 #pragma unroll
-            for (int v = 0; v < 4; ++v) {
-                const int row = rt * 16 + 4 * lq + v;
-                const int64_t t = s_orow[row];
-                if (t < 0) continue;
-                const float wgt = s_w[row];
-                const int64_t dst = t * g.N + n0 + jt * 256 + 64 * wv + lr;
+                for (int v = 0; v < 4; ++v) {
+                    const int row = rt * 16 + 4 * lq + v;
+                    const int64_t t = s_orow[row];
+                    if (t < 0) continue;
+                    const float wgt = s_w[row];
+                    const int64_t dst = t * g.N + n0 + jt * 256 + 64 * wv + lr;
 #pragma unroll
-                for (int ct = 0; ct < kNCT; ++ct)
-                    acc_add(g.acc, g.acc_dtype, dst + 16 * ct, acc[rt][ct][v] * wgt);
+                    for (int ct = 0; ct < kNCT; ++ct) add(dst, 16 * ct, acc[rt][ct][v] * wgt);
+                }
+        };
+        if (ACC32)
+            rows([&](int64_t i, int o, float y) {
+                unsafeAtomicAdd(reinterpret_cast<float*>(g.acc) + i + o, y);
+            });
+        else
+            rows([&](int64_t i, int o, float y) { acc_add(g.acc, g.acc_dtype, i + o, y); });
+    };
+
+    // The K loop, a copy for weights that this M-block alone reads (non-temporal
+    // loads: they should displace nothing) and one for weights it shares with
+    // the expert's other M-blocks. Measured on MI355X, MiMo dims: with
+    // non-temporal loads throughout, blocks of one expert each read its weights
+    // from HBM (skewed routing, 16-row blocks, T=256: 610 us, 428 with the two
+    // copies); with ordinary loads throughout, uniform routing T=256 ran 1163
+    // us instead of 1050.
+    auto k_loop = [&](auto once) __attribute__((always_inline)) {
+    constexpr bool ONCE = decltype(once)::value;
+    constexpr int WPOL = ONCE ? 2 : 0;             // buffer cache policy: nt
+    // operands of K block kb of column group jt
+    auto load = [&](Step<NRT, W4>& s, int kb, int jt) __attribute__((always_inline)) {
+        const int so = __builtin_amdgcn_readfirstlane(kb * BSTEP + jt * (256 * KBY));
+#pragma unroll
+        for (int ct = 0; ct < kNCT; ++ct) {
+            const __amdgpu_buffer_rsrc_t r = rb[G1 ? ct >> 1 : 0];
+            s.b[ct][0] = __builtin_amdgcn_raw_buffer_load_b128(r, boff[ct], so, WPOL);
+            if (!W4)
+                s.b[ct][W4 ? 0 : 1] =
+                    __builtin_amdgcn_raw_buffer_load_b128(r, boff[ct] + BHI, so, WPOL);
+        }
+        // XQ: A comes from LDS when the step is computed (no registers held)
+        if constexpr (!XQ) {
+#pragma unroll
+            for (int rt = 0; rt < NRT; ++rt) {
+                const uint8_t* p = asrc[rt] + kb * 128;
+                s.a[rt][0] = *reinterpret_cast<const v4i*>(p);
+                s.a[rt][1] = *reinterpret_cast<const v4i*>(p + AHI);
             }
+        }
     };
 
     // stage 1: K step k of the walk is K block km(k), the walk rotated by a
     // per-workgroup multiple of D so that concurrent workgroups stream
     // different offsets of their weight rows
-    const int krot = G1 && g.krot ? D * (int)((blockIdx.x * 5u + blockIdx.y * 3u) % (KBS / D)) : 0;
+    // (M-blocks that share weights walk in step, so that one's loads are the
+    // others' L2 hits)
+    const int krot =
+        G1 && g.krot ? D * (int)(((unsigned)bx * 5u + (unsigned)(ONCE ? mb : e) * 3u) % (KBS / D)) : 0;
     auto km = [&](int k) {
         int r = k - kbeg + krot;
         if (r >= KBS) r -= KBS;
@@ -426,6 +524,48 @@ __global__ __launch_bounds__(kThreads) void moe_gemm_stream_kernel(Args g) {
         }
 #pragma unroll
         for (int d = 0; d < D; ++d) compute(buf[d], km(kend - D + d), 0, sgc, d);
+    } else {
+        // ---- K loop over ntw * KB steps: D steps in flight; a group's last
+        // steps are followed by its epilogue while the next group's first D
+        // steps load (D divides KB) ----
+        const int KBT = KB * ntw;
+        int kbl = 0, jt = 0;                   // K block and column group of step kb0
+        for (int kb0 = 0; kb0 < KBT - D; kb0 += D) {
+            // K block and group of step kb0 + D
+            int kbn = kbl + D, jn = jt;
+            if (kbn == KB) {
+                kbn = 0;
+                ++jn;
+            }
+            if (W4) load_sg(sgn, kbn, jn);
+#pragma unroll
+            for (int d = 0; d < D; ++d) {
+                compute(buf[d], kbl + d, jt, sgc, d);
+                load(buf[d], kbn + d, jn);
+            }
+            next_scales();
+            if (jn != jt) {
+                epilogue2(jt);
+#pragma unroll
+                for (int rt = 0; rt < NRT; ++rt)
+#pragma unroll
+                    for (int ct = 0; ct < kNCT; ++ct) acc[rt][ct] = v4f{0.f, 0.f, 0.f, 0.f};
+            }
+            kbl = kbn;
+            jt = jn;
+        }
+#pragma unroll
+        for (int d = 0; d < D; ++d) compute(buf[d], kbl + d, jt, sgc, d);
+        epilogue2(jt);
+    }
+    };
+    if (shared_w)
+        k_loop(std::false_type{});
+    else
+        k_loop(std::true_type{});
+    if constexpr (STAGE == 2) return;
+
+    if constexpr (G1) {
         if constexpr (!FUSED) {
             if (g.out_mode == kOutGateUp) {
                 // ---- fp32 gate | up rows before the activation; a K range of
@@ -469,7 +609,7 @@ __global__ __launch_bounds__(kThreads) void moe_gemm_stream_kernel(Args g) {
             // whole L2 in every workgroup.
             constexpr int NP = NRT * kNCT;                 // v4f per thread
             constexpr int kSc1 = 16;                       // buffer cache policy: sc1
-            const int64_t tile = (int64_t)mb * (gridDim.x / S) + nt;
+            const int64_t tile = (int64_t)mb * (g.gx / S) + nt;
             const __amdgpu_buffer_rsrc_t rp = __builtin_amdgcn_make_buffer_rsrc(
                 g.kpart + tile * S * NP * kThreads, (short)0, S * NP * kThreads * 16, 0x00020000);
 #pragma unroll
@@ -501,40 +641,6 @@ __global__ __launch_bounds__(kThreads) void moe_gemm_stream_kernel(Args g) {
             if (tid == 0)                                  // zero again for the next call
                 __hip_atomic_store(&g.kcnt[tile], 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
         }
-    } else {
-        // ---- K loop over ntw * KB steps: D steps in flight; a group's last
-        // steps are followed by its epilogue while the next group's first D
-        // steps load (D divides KB) ----
-        const int KBT = KB * ntw;
-        int kbl = 0, jt = 0;                   // K block and column group of step kb0
-        for (int kb0 = 0; kb0 < KBT - D; kb0 += D) {
-            // K block and group of step kb0 + D
-            int kbn = kbl + D, jn = jt;
-            if (kbn == KB) {
-                kbn = 0;
-                ++jn;
-            }
-            if (W4) load_sg(sgn, kbn, jn);
-#pragma unroll
-            for (int d = 0; d < D; ++d) {
-                compute(buf[d], kbl + d, jt, sgc, d);
-                load(buf[d], kbn + d, jn);
-            }
-            next_scales();
-            if (jn != jt) {
-                epilogue2(jt);
-#pragma unroll
-                for (int rt = 0; rt < NRT; ++rt)
-#pragma unroll
-                    for (int ct = 0; ct < kNCT; ++ct) acc[rt][ct] = v4f{0.f, 0.f, 0.f, 0.f};
-            }
-            kbl = kbn;
-            jt = jn;
-        }
-#pragma unroll
-        for (int d = 0; d < D; ++d) compute(buf[d], kbl + d, jt, sgc, d);
-        epilogue2(jt);
-        return;
     }
 
     // ---- fused: the down GEMM's weight sources; its first D2 column groups
@@ -579,7 +685,7 @@ __global__ __launch_bounds__(kThreads) void moe_gemm_stream_kernel(Args g) {
     };
     // column group of walk position p (rotated like stage 1's K walk)
     const int grot =
-        FUSED && g.krot ? (int)((blockIdx.x * 5u + blockIdx.y * 3u) % (unsigned)NG) : 0;
+        FUSED && g.krot ? (int)(((unsigned)bx * 5u + (unsigned)mb * 3u) % (unsigned)NG) : 0;
     auto gm = [&](int p) { return p + grot < NG ? p + grot : p + grot - NG; };
     B2 bq[D2];
 #pragma unroll
@@ -741,27 +847,36 @@ constexpr int max_depth() { return BM == 16 ? 4 : 2; }
 template <int BM, int STAGE, bool SHUFFLED, bool W4, bool XQ = false>
 static void launch_depth(int KB, dim3 grid, const Args& a, hipStream_t s) {
     constexpr int DM = max_depth<BM>();
+    auto go = [&](auto depth) {
+        constexpr int D = decltype(depth)::value;
+        if constexpr (STAGE == 2) {
+            if (a.acc_dtype != DT_FP32) {
+                hipLaunchKernelGGL(
+                    (moe_gemm_stream_kernel<BM, STAGE, SHUFFLED, W4, D, XQ, false>), grid,
+                    dim3(kThreads), 0, s, a);
+                return;
+            }
+        }
+        hipLaunchKernelGGL((moe_gemm_stream_kernel<BM, STAGE, SHUFFLED, W4, D, XQ>), grid,
+                           dim3(kThreads), 0, s, a);
+    };
     // One-token MXFP4 stage 1 (XQ: A from LDS, so a step holds only weight
     // fragments, 16 bytes per lane and column tile) keeps 8 steps in flight.
     // Measured on MI355X at MiMo T=1, alternating: A8W4 layer 30.6-30.8 ->
     // 30.0-30.1 us; FP8 at 8 steps (256 VGPRs + 60 AGPRs, one workgroup per
     // CU) was slower, 43.4-43.5 -> 43.9-44.0 us, so FP8 keeps 4.
     if constexpr (XQ && W4) {
-        if (KB % 8 == 0) {
-            hipLaunchKernelGGL((moe_gemm_stream_kernel<BM, STAGE, SHUFFLED, W4, 8, XQ>), grid,
-                               dim3(kThreads), 0, s, a);
-            return;
-        }
+        if (KB % 8 == 0) return go(std::integral_constant<int, 8>{});
     }
-    if (DM >= 4 && KB % 4 == 0)
-        hipLaunchKernelGGL((moe_gemm_stream_kernel<BM, STAGE, SHUFFLED, W4, DM >= 4 ? 4 : 2, XQ>),
-                           grid, dim3(kThreads), 0, s, a);
-    else if (KB % 2 == 0)
-        hipLaunchKernelGGL((moe_gemm_stream_kernel<BM, STAGE, SHUFFLED, W4, 2, XQ>), grid,
-                           dim3(kThreads), 0, s, a);
-    else
-        hipLaunchKernelGGL((moe_gemm_stream_kernel<BM, STAGE, SHUFFLED, W4, 1, XQ>), grid,
-                           dim3(kThreads), 0, s, a);
+    // three steps of stage 2's K ranges that four do not divide (inter 384,
+    // 768: 3 and 6 steps, which ran one and two at a time)
+    if constexpr (DM >= 4) {
+        if (KB % 4 == 0) return go(std::integral_constant<int, 4>{});
+        if constexpr (STAGE == 2)
+            if (KB % 3 == 0) return go(std::integral_constant<int, 3>{});
+    }
+    if (KB % 2 == 0) return go(std::integral_constant<int, 2>{});
+    go(std::integral_constant<int, 1>{});
 }
 
 template <int STAGE, bool SHUFFLED, bool W4>
@@ -782,8 +897,13 @@ static void launch_bm(int bm, int KB, dim3 grid, const Args& a, hipStream_t s) {
         AMD_CHECK(false, "streaming GEMM block_m must be 16 or 32");
 }
 
+// gx column tiles (x K ranges) by mblocks M-blocks.
 template <int STAGE>
-static void launch(int bm, int KB, dim3 grid, const Args& a, int shuffled, hipStream_t s) {
+static void launch(int bm, int KB, int64_t gx, int64_t mblocks, Args a, int shuffled,
+                   hipStream_t s) {
+    a.gx = (int)gx;
+    AMD_CHECK(gx * mblocks < (int64_t(1) << 31), "too many M-blocks");
+    const dim3 grid((unsigned)gx, (unsigned)mblocks);
     const bool w4 = a.w_scale8 != nullptr;
     if (w4) {
         if (shuffled)
@@ -798,40 +918,14 @@ static void launch(int bm, int KB, dim3 grid, const Args& a, int shuffled, hipSt
     }
 }
 
-// Stage 2's 256-column groups per workgroup. A stage-2 workgroup streams
-// 256 x K weight bytes per group (MiMo dims: 512 KB fp8, 256 KB fp4, against
-// a stage-1 workgroup's 1 MB / 512 KB), so its setup and epilogue weigh more;
-// walking groups in one K loop, up to ~1 MB of weights per workgroup, evens
-// that out while the grid stays large enough to keep every CU streaming.
-// Measured on MI355X (stage 2, MiMo dims): fp8 T=32 231 -> 213 us at two
-// groups, T=128 378 -> 351 us; fp4 T=32 128 -> 124 us at four; T=1 15 ->
-// 24 us at two (64 workgroups), hence the grid floor. est_blocks: the
-// expected M-blocks (at decode sizes one per touched expert).
-// fp8 weights follow a table of the single-walk grid's rounds r1 (est_blocks
-// x groups / 512 workgroup slots), measured on MI355X at MiMo dims (stage 2,
-// us at one / two / four groups): T=8 (r1 = 2) 81.7 / 78.2 / 81.5, T=16
-// (r1 = 4) 151 / 148 / 139, T=32 (r1 = 8) 237 / 217 / 222, T=128 (r1 = 32)
-// 377 / 352 / 343 -- a walk that leaves one full round wins, and larger
-// grids prefer two groups up to ~24 rounds, four beyond.
-// AITER_AMD_ST_NTW2 forces a count (tests use it).
-static int pick_ntw2(int64_t groups, int64_t KB, int64_t KBY, int64_t est_blocks) {
+// AITER_AMD_ST_NTW2 forces stage 2's column groups per workgroup (tests use
+// it); 0: the kernel picks (walk_groups).
+static int forced_ntw2(int64_t groups, int64_t KB) {
     if (const char* env = getenv("AITER_AMD_ST_NTW2")) {
         const int c = atoi(env);
         if (c >= 1 && groups % c == 0 && c * KB <= kMaxKB) return c;
     }
-    if (KBY == KB * 128) {   // fp8 weights
-        const int64_t w1 = est_blocks * groups;     // workgroups of the single walk
-        int c = w1 >= 24 * 512 ? 4 : w1 >= 6 * 512 ? 2 : w1 >= 3 * 512 ? 4 : w1 >= 768 ? 2 : 1;
-        while (c > 1 && (groups % c != 0 || c * KB > kMaxKB)) c /= 2;
-        return c;
-    }
-    constexpr int64_t kMinWgs = 1024;             // 256 CUs x 2 workgroups x 2 rounds
-    constexpr int64_t kTargetBytes = 1 << 20;     // weight bytes per workgroup
-    for (int64_t c = std::max<int64_t>(1, kTargetBytes / (256 * KBY)); c > 1; c /= 2) {
-        if (groups % c == 0 && c * KB <= kMaxKB && est_blocks * groups / c >= kMinWgs)
-            return (int)c;
-    }
-    return 1;
+    return 0;
 }
 
 // Stage-1 split-K: K ranges per column tile. Measured on MI355X at MiMo
@@ -1208,8 +1302,8 @@ void launch_moe_stage1_stream(const uint8_t* a, const float* a_scale, int64_t sa
     if (max_m_blocks == 0) return;
     // split-K: only the M-blocks the partial buffers cover can hold routed rows
     const int64_t mblocks = g.ksplit > 1 ? g.kmb : max_m_blocks;
-    const dim3 grid((unsigned)(inter / 128 * g.ksplit), (unsigned)mblocks);
-    stream::launch<1>((int)block_m, (int)(K / 128 / g.ksplit), grid, g, shuffled, stream);
+    stream::launch<1>((int)block_m, (int)(K / 128 / g.ksplit), inter / 128 * g.ksplit, mblocks, g,
+                      shuffled, stream);
     AMD_HIP_CHECK(hipGetLastError());
 }
 
@@ -1266,8 +1360,7 @@ void launch_moe_stage1_stream_rows(const uint8_t* a, const float* a_scale, int64
     g.E = (int)E;
     g.a_rows = a_rows;
     if (max_m_blocks == 0) return;
-    const dim3 grid((unsigned)(inter / 128 * S), (unsigned)(max_m_blocks << shift));
-    stream::launch<1>(bmk, KB / S, grid, g, shuffled, stream);
+    stream::launch<1>(bmk, KB / S, inter / 128 * S, max_m_blocks << shift, g, shuffled, stream);
     AMD_HIP_CHECK(hipGetLastError());
 }
 
@@ -1299,10 +1392,9 @@ void launch_moe_stage2_stream(const uint8_t* a2, const float* a2_scale, const ui
     g.E = (int)E;
     g.a_rows = a_rows;
     if (max_m_blocks == 0) return;
-    g.ntw = stream::pick_ntw2(hidden / 256, inter / 128, w2_scale_e8m0 ? inter / 2 : inter,
-                              std::min<int64_t>(a_rows, E));
-    const dim3 grid((unsigned)(hidden / 256 / g.ntw), (unsigned)max_m_blocks);
-    stream::launch<2>((int)block_m, (int)(inter / 128), grid, g, shuffled, stream);
+    g.ntw = stream::forced_ntw2(hidden / 256, inter / 128);
+    stream::launch<2>((int)block_m, (int)(inter / 128), hidden / 256, max_m_blocks, g,
+                      shuffled, stream);
     AMD_HIP_CHECK(hipGetLastError());
 }
 
@@ -1365,8 +1457,8 @@ void launch_moe_fused_stream(const uint8_t* a, const float* a_scale, int64_t sa_
     g.a_rows = a_rows;
     if (max_m_blocks == 0) return;
     const int64_t mblocks = g.ksplit > 1 ? g.kmb : max_m_blocks;
-    const dim3 grid((unsigned)(inter / 128 * g.ksplit), (unsigned)mblocks);
-    stream::launch<3>((int)block_m, (int)(hidden / 128 / g.ksplit), grid, g, shuffled, stream);
+    stream::launch<3>((int)block_m, (int)(hidden / 128 / g.ksplit), inter / 128 * g.ksplit, mblocks,
+                      g, shuffled, stream);
     AMD_HIP_CHECK(hipGetLastError());
 }
 

@@ -1098,3 +1098,47 @@ def test_prequant_layer_beyond_the_row_limit(cuda_device):
                                 a1_scale=a1s[:n], block_size_M=64).float()
     a, b = run(T)[:T - 1], run(T - 1)
     assert ((a - b).abs() <= b.abs() * 2.0 ** -7 + 8 * 2.0 ** -23 * b.abs().max() * 8).all()
+
+
+# column-tile counts that 8 divides and that it does not (stage 1 inter / 128,
+# stage 2 model_dim / 256 over the groups a workgroup walks), M-blocks below, at
+# and above the 32 of a whole round of groups, K-step counts of 1, 2, 3, 5, 6 and
+# 8 in stage 2, experts with one M-block and with many
+@pytest.mark.parametrize("weights", ["fp8", "mxfp4"])
+@pytest.mark.parametrize("bm", [16, 32])
+@pytest.mark.parametrize("tokens,H,I,E", [
+    (7, 512, 128, 3), (40, 1792, 256, 5), (150, 768, 384, 6), (400, 1792, 384, 9),
+    (260, 512, 640, 40), (333, 2048, 768, 33), (512, 1024, 1024, 8), (90, 3584, 256, 64)])
+def test_stream_shared_weights_and_tile_order(cuda_device, monkeypatch, weights, bm, tokens, H, I,
+                                              E):
+    """The stream kernel's workgroup order, column walks and weight-load
+    policies against the prefill kernels (64-row blocks), which pass the oracle
+    tests: with the staggered K walk off both sum K blocks in the same order,
+    so stage 1 is bit for bit the same and a pair's stage-2 row too; a token's
+    pairs then add in any order, (k - 1) * 2^-24 of the sum of their magnitudes."""
+    monkeypatch.setenv("AITER_AMD_ST_ROT", "0")
+    k = min(3, E)
+    cfg = W.MoEConfig("order", tokens, H, I, E, k, seed=tokens, weights=weights, routing="zipf",
+                      zipf_s=1.5)
+    wts = W.make_weights(cfg, device=cuda_device)
+    tw, ids = W.make_routing(cfg, device=cuda_device)
+    a1, a1s = A.per_group_quant_hip(W.make_hidden(cfg, device=cuda_device))
+    st1, st2 = ((A.moe_stage1_a8w4, A.moe_stage2_a8w4) if weights == "mxfp4" else
+                (A.moe_stage1_fp8_blockscale, A.moe_stage2_fp8_blockscale))
+    monkeypatch.setenv("AITER_AMD_W4_PF_ROWS1", "0")     # MXFP4 on the prefill kernels too
+    monkeypatch.setenv("AITER_AMD_W4_PF_ROWS2", "0")
+    got = {}
+    for b, dt in ((64, torch.float32), (bm, torch.float32), (bm, torch.bfloat16)):
+        sid, sw, seid, nv, acc = A.moe_sorting(ids, tw, E, H, dt, b)
+        a2, a2s = st1(a1, a1s, wts["w1"], wts["w1_scale"], sid, seid, nv, k, b, True)
+        st2(a2, a2s, wts["w2"], wts["w2_scale"], sid, sw, seid, nv, acc, b, True)
+        got[b, dt] = a2, a2s, acc
+    (ra2, rs, racc), (a2, a2s, acc) = got[64, torch.float32], got[bm, torch.float32]
+    assert torch.equal(a2s, rs)
+    assert torch.equal(a2.view(torch.uint8), ra2.view(torch.uint8))
+    # (terms that cancel may each be a few times the largest sum)
+    tol = 4 * k * 2.0 ** -23 * racc.abs().max()
+    assert ((acc - racc).abs() <= tol).all()
+    # a bf16 moe_buf rounds after every add: half a spacing, 2^-8, per pair
+    b16 = got[bm, torch.bfloat16][2].float()
+    assert ((b16 - racc).abs() <= 2 * k * 2.0 ** -8 * racc.abs().max()).all()
