@@ -258,13 +258,17 @@ __global__ __launch_bounds__(kThreads, 2) void moe_gemm_prefill_kernel(Args g) {
     const int srow0 = mb * g.block_m + (mt % subs) * BM; // first sorted row of the tile
     if (srow0 >= nvalid) return;
     const int tokens = g.num_valid[1];
+    // the tile's expert and its rows' pairs and weights, all in flight at once
     const int e = g.sorted_eids[mb];
+    const int r0 = tid < BM ? tid : 0;
+    const uint32_t id = (uint32_t)g.sorted_ids[srow0 + r0];
+    const float route_w = g.sorted_w ? g.sorted_w[srow0 + r0] : 1.0f;
     if (e < 0 || e >= g.E) return;
     const int n0 = nt * ntw * TROWS;                     // first column of the first tile
 
     int any_valid = 0;
-    for (int r = tid; r < BM; r += kThreads) {
-        const uint32_t id = (uint32_t)g.sorted_ids[srow0 + r];
+    if (tid < BM) {
+        const int r = tid;
         const int t = (int)(id & 0xFFFFFFu);
         const int s = (int)(id >> 24);
         const bool valid = t < tokens && s < g.topk;
@@ -279,8 +283,8 @@ __global__ __launch_bounds__(kThreads, 2) void moe_gemm_prefill_kernel(Args g) {
         s_orow[r] = orow;
         // routing weight of the pair (1 when none is passed: stage 2 without
         // weights, or stage 1 without doweight); stage 1 applies it only when given
-        s_w[r] = valid ? (g.sorted_w ? g.sorted_w[srow0 + r] : 1.0f) : 0.0f;
-        any_valid |= (int)valid;
+        s_w[r] = valid ? route_w : 0.0f;
+        any_valid = (int)valid;
     }
     // a tile whose rows are all padding (the end of an expert's last
     // M-block) has nothing to compute
