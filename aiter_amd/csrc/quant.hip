@@ -227,64 +227,73 @@ __global__ __launch_bounds__(256) void slot_sum_kernel(const TP* __restrict__ pa
     }
 }
 
-// slot_sum_wave_kernel: one token per wave, four per workgroup, so the short
-// id -> mask -> row chains of an expert-parallel share's rows (about one
-// routed slot in eight) overlap. Each lane holds kPieces 8-column pieces of
-// the row (a 4096-column row in one pass) and, slot by slot in slot order,
-// issues all of a slot's piece loads before summing them. Measured on MI355X,
-// EP share (32 of 256 experts, 64-row blocks): T=4096 20.0 -> 18.9 us, T=2048
-// 14.7 -> 13.7 us against two pieces per pass (the per-workgroup kernel took
-// 21 us); 4 pieces per lane (two passes, 92 instead of 168 VGPRs) 20.5 us.
+// slot_sum_wave_kernel: a wave per token and span of 2048 columns (1024 of fp32
+// rows), four waves per workgroup, for an expert-parallel share's rows (about
+// one routed slot in eight). What bounds it is the chain id -> mask -> row ->
+// store, so many short waves run side by side: a lane holds four (two) 8-column
+// pieces, the token count is loaded beside the ids, and two slots' pieces are in
+// flight before either is summed, in slot order. Measured on MI355X, EP share
+// (32 of 256 experts), hidden 4096, against a wave per whole row, medians
+// of 20: T=4096 22.6 -> 20.7 us, T=2048 12.7 -> 12.2, fp32 rows T=4096 39.8 -> 36.7.
 template <bool kBf16, typename TP>
 __global__ __launch_bounds__(256) void slot_sum_wave_kernel(
     const TP* __restrict__ part, const int32_t* __restrict__ topk_ids,
     const int32_t* __restrict__ mask, int num_experts, const int32_t* __restrict__ num_valid,
     uint16_t* out, int64_t rows, int topk, int cols, const uint16_t* addend) {
-    constexpr int kPieces = 16 / sizeof(TP);             // 4 of fp32 rows: the same bytes in flight
-    int64_t tokens = (int64_t)num_valid[1];
-    tokens = tokens < rows ? tokens : rows;
+    constexpr int kPieces = 8 / sizeof(TP);
     const int c8 = cols / 8;
     const int lane = threadIdx.x & 63;
-    for (int64_t t = (int64_t)blockIdx.x * 4 + (threadIdx.x >> 6); t < tokens;
-         t += (int64_t)gridDim.x * 4) {
+    const int spans = (c8 + 64 * kPieces - 1) / (64 * kPieces);
+    for (int64_t q = (int64_t)blockIdx.x * 4 + (threadIdx.x >> 6); q < rows * spans;
+         q += (int64_t)gridDim.x * 4) {
+        const int64_t t = q / spans;
+        const int base = (int)(q - t * spans) * 64 * kPieces + lane;
         int ok = 0;
         if (lane < topk) {
             const int id = topk_ids[t * topk + lane];
             ok = id >= 0 && id < num_experts && (!mask || mask[id] != 0);
         }
-        const uint32_t valid = (uint32_t)__builtin_amdgcn_ballot_w64(ok);
+        uint32_t m = (uint32_t)__builtin_amdgcn_ballot_w64(ok);
+        if (t >= (int64_t)num_valid[1]) continue;
         const TP* src = part + t * topk * (int64_t)cols;
-        for (int base = lane; base < c8; base += 64 * kPieces) {
-            float a[kPieces][8] = {};
-            uint32_t m = valid;
-            while (m != 0) {
-                const int j = __builtin_ctz(m);
-                m &= m - 1;
-                Row8<TP> v[kPieces];
-#pragma unroll
-                for (int i = 0; i < kPieces; ++i) {
-                    const int cc = base + 64 * i;
-                    v[i].clear();
-                    if (cc < c8) v[i].load(src + (int64_t)j * cols + cc * 8);
-                }
-#pragma unroll
-                for (int i = 0; i < kPieces; ++i) v[i].add_to(a[i]);
-            }
+        float a[kPieces][8] = {};
+        while (m != 0) {
+            const int j0 = __builtin_ctz(m);
+            m &= m - 1;
+            const bool two = m != 0;
+            const int j1 = two ? __builtin_ctz(m) : j0;
+            m &= m - 1;
+            Row8<TP> v0[kPieces], v1[kPieces];
 #pragma unroll
             for (int i = 0; i < kPieces; ++i) {
                 const int cc = base + 64 * i;
-                if (cc >= c8) continue;
-                if (addend) add_row8<kBf16>(a[i], addend + t * cols + cc * 8);
-                uint32_t w[4];
-#pragma unroll
-                for (int e = 0; e < 4; ++e)
-                    w[e] = kBf16 ? f32_to_bf16_bits(a[i][2 * e]) |
-                                       ((uint32_t)f32_to_bf16_bits(a[i][2 * e + 1]) << 16)
-                                 : f32_to_fp16_bits(a[i][2 * e]) |
-                                       ((uint32_t)f32_to_fp16_bits(a[i][2 * e + 1]) << 16);
-                *reinterpret_cast<v4i*>(out + t * cols + cc * 8) =
-                    v4i{(int)w[0], (int)w[1], (int)w[2], (int)w[3]};
+                v0[i].clear();
+                v1[i].clear();
+                if (cc < c8) {
+                    v0[i].load(src + (int64_t)j0 * cols + cc * 8);
+                    if (two) v1[i].load(src + (int64_t)j1 * cols + cc * 8);
+                }
             }
+#pragma unroll
+            for (int i = 0; i < kPieces; ++i) {
+                v0[i].add_to(a[i]);
+                if (two) v1[i].add_to(a[i]);
+            }
+        }
+#pragma unroll
+        for (int i = 0; i < kPieces; ++i) {
+            const int cc = base + 64 * i;
+            if (cc >= c8) continue;
+            if (addend) add_row8<kBf16>(a[i], addend + t * cols + cc * 8);
+            uint32_t w[4];
+#pragma unroll
+            for (int e = 0; e < 4; ++e)
+                w[e] = kBf16 ? f32_to_bf16_bits(a[i][2 * e]) |
+                                   ((uint32_t)f32_to_bf16_bits(a[i][2 * e + 1]) << 16)
+                             : f32_to_fp16_bits(a[i][2 * e]) |
+                                   ((uint32_t)f32_to_fp16_bits(a[i][2 * e + 1]) << 16);
+            *reinterpret_cast<v4i*>(out + t * cols + cc * 8) =
+                v4i{(int)w[0], (int)w[1], (int)w[2], (int)w[3]};
         }
     }
 }
@@ -296,7 +305,9 @@ void launch_slot_sum(const void* part, int part_dtype, const int32_t* topk_ids,
     if (rows == 0 || cols == 0) return;
     // an expert mask means an expert-parallel share: most slots are not routed here
     const bool per_wave = mask != nullptr;
-    const int blocks = (int)std::min<int64_t>(ceil_div(rows, per_wave ? 4 : 1), 8192);
+    const int64_t spans = ceil_div(cols, 64 * 64 / (part_dtype == DT_FP32 ? 4 : 2));
+    const int blocks =
+        (int)std::min<int64_t>(per_wave ? ceil_div(rows * spans, 4) : rows, per_wave ? 65536 : 8192);
     auto go = [&](auto kern, auto* rows_of_pairs) {
         hipLaunchKernelGGL(kern, dim3(blocks), dim3(256), 0, stream, rows_of_pairs, topk_ids, mask,
                            (int)num_experts, num_valid, (uint16_t*)out, rows, (int)topk,

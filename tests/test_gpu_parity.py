@@ -1142,3 +1142,31 @@ def test_stream_shared_weights_and_tile_order(cuda_device, monkeypatch, weights,
     # a bf16 moe_buf rounds after every add: half a spacing, 2^-8, per pair
     b16 = got[bm, torch.bfloat16][2].float()
     assert ((b16 - racc).abs() <= 2 * k * 2.0 ** -8 * racc.abs().max()).all()
+
+
+@pytest.mark.parametrize("H", [256, 1792, 2048, 2304, 4096, 7168])
+@pytest.mark.parametrize("prequant", [False, True])   # bf16 and fp32 per-pair rows
+def test_slot_sum_wave_spans(cuda_device, H, prequant):
+    """The expert-parallel slot sum (a wave per span of a row) against the dense
+    one: with every expert local both add the same rows in slot order, so the
+    outputs are equal bit for bit; with some masked, a token without a local
+    expert gets a zero row."""
+    cfg = W.MoEConfig("spans", 131, H, 128, 8, 5, seed=H)
+    wts = W.make_weights(cfg, device=cuda_device)
+    tw, ids = W.make_routing(cfg, device=cuda_device)
+    x = W.make_hidden(cfg, device=cuda_device)
+    kw = dict(w1_scale=wts["w1_scale"], w2_scale=wts["w2_scale"], block_size_M=64)
+    if prequant:
+        x, kw["a1_scale"] = A.per_group_quant_hip(x)
+    run = lambda **k: W.run_layer("fp8", x, wts["w1"], wts["w2"], tw, ids, **kw, **k)
+    dense = run()
+    assert torch.equal(run(expert_mask=torch.ones(8, dtype=torch.int32, device=cuda_device)), dense)
+    n = torch.tensor([77], dtype=torch.int32, device=cuda_device)
+    ones = torch.ones(8, dtype=torch.int32, device=cuda_device)
+    assert torch.equal(run(expert_mask=ones, num_local_tokens=n)[:77], dense[:77])
+    away = torch.full_like(ids, 11)                   # experts 8 .. 15 live on another GPU
+    mixed = torch.where((torch.arange(131, device=cuda_device) % 3 == 0)[:, None], away, ids)
+    mask = (torch.arange(16, device=cuda_device) < 8).to(torch.int32)
+    got = W.run_layer("fp8", x, wts["w1"], wts["w2"], tw, mixed, expert_mask=mask, **kw)
+    assert torch.count_nonzero(got[::3]) == 0
+    assert torch.equal(got[1::3], dense[1::3]) and torch.equal(got[2::3], dense[2::3])
