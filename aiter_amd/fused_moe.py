@@ -220,18 +220,12 @@ def fused_moe(
     """Same signature and result as aiter.fused_moe.fused_moe (fused_moe.py:118-169);
     runs the registered custom op torch.ops.aiter_amd.fused_moe_ as the reference
     runs torch.ops.aiter.fused_moe_ (fused_moe.py:172-205)."""
-    return _layer_op()(
+    return _LAYER_OP(
         hidden_states, w1, w2, topk_weight, topk_ids, expert_mask, int(activation),
         int(quant_type), bool(doweight_stage1), w1_scale, w2_scale, a1_scale, a2_scale,
         int(block_size_M) if block_size_M else -1, num_local_tokens,
         int(moe_sorting_dispatch_policy), dtype, int(hidden_pad), int(intermediate_pad), bias1,
         bias2)
-
-
-@functools.lru_cache(maxsize=1)
-def _layer_op():
-    # the overload itself: the packet would resolve it on every call
-    return torch.ops.aiter_amd.fused_moe_.default
 
 
 def fused_moe_a8w4(
@@ -560,6 +554,9 @@ def _register_custom_op():
 
 
 _register_custom_op()
+# the overload itself: the packet would resolve it on every call. A plain global,
+# which torch.compile traces without a warning (a cached getter draws one).
+_LAYER_OP = torch.ops.aiter_amd.fused_moe_.default
 
 
 def _stage1(entry, a1, a1_scale, w1, w1_scale, sorted_ids, sorted_expert_ids, num_valid_ids,

@@ -317,6 +317,37 @@ def test_fused_moe_is_a_registered_custom_op():
         assert out.shape == (6, 256) and out.dtype == torch.float16
 
 
+def test_fused_moe_compiles_without_a_warning():
+    """fused_moe traces into one full graph of the custom op, and tracing warns
+    of nothing."""
+    import warnings
+
+    graphs = []
+
+    def backend(gm, _):
+        graphs.append(gm.graph)
+        return lambda *a: (torch.zeros(4, 256, dtype=torch.bfloat16),)
+
+    fp8 = torch.float8_e4m3fn
+    args = (torch.zeros(4, 256, dtype=torch.bfloat16), torch.zeros(2, 256, 256, dtype=fp8),
+            torch.zeros(2, 256, 128, dtype=fp8), torch.ones(4, 2),
+            torch.zeros(4, 2, dtype=torch.int32), torch.ones(2, 2, 2), torch.ones(2, 2, 1))
+
+    def layer(x, w1, w2, tw, ids, s1, s2):
+        return A.fused_moe(x, w1, w2, tw, ids, quant_type=A.QuantType.per_128x128, w1_scale=s1,
+                           w2_scale=s2)
+
+    torch._dynamo.reset()
+    with warnings.catch_warnings(record=True) as seen:
+        warnings.simplefilter("always")
+        out = torch.compile(layer, fullgraph=True, backend=backend)(*args)
+    torch._dynamo.reset()
+    assert out.shape == (4, 256) and len(graphs) == 1
+    assert sum("fused_moe_" in str(n.target) for n in graphs[0].nodes) == 1
+    assert [str(w.message) for w in seen if "aiter_amd" in str(w.message) or
+            "lru_cache" in str(w.message)] == []
+
+
 def test_enum_values_match_reference():
     from aiter_amd import ActivationType, QuantType
 
