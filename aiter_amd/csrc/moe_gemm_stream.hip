@@ -100,6 +100,7 @@ struct Args {
     // 64- or 128-row M-blocks are walked as 32-row ones
     int eid_shift;
     int gx;                    // stage 1: column tiles x ksplit; stage 2: 256-column groups
+    int mblocks;               // M-blocks that sorted_eids has an entry for and the grid covers
     // direct M-blocks, for a layer too small to be worth a sorting launch:
     // with dir_ids set, M-block p holds routing pair p = token * topk + slot
     // of dir_tokens tokens in its first row (the rest is padding), its expert
@@ -206,7 +207,8 @@ __global__ __launch_bounds__(kThreads) void moe_gemm_stream_kernel(Args g) {
     const int nvalid = direct ? g.dir_tokens * g.topk * BM : g.num_valid[0];
     // (column tile x K range, M-block) of the workgroup; stage 2 walks ntw
     // consecutive 256-column groups in one K loop (steps s = jt * KB + kb)
-    const int mv = (nvalid + BM - 1) / BM;
+    // M-blocks to run: the routed ones, as far as the caller's metadata goes
+    const int mv = min((nvalid + BM - 1) / BM, g.mblocks);
     const int ntw = STAGE != 2 ? 1 : g.ntw > 0 ? g.ntw : walk_groups<W4>(mv, g.gx, g.K / 128);
     int bx = blockIdx.x, mb = blockIdx.y;
     if (ntw > 1 || ((g.gx & 7) != 0 && mv >= 32))
@@ -902,6 +904,7 @@ template <int STAGE>
 static void launch(int bm, int KB, int64_t gx, int64_t mblocks, Args a, int shuffled,
                    hipStream_t s) {
     a.gx = (int)gx;
+    a.mblocks = (int)mblocks;
     AMD_CHECK(gx * mblocks < (int64_t(1) << 31), "too many M-blocks");
     const dim3 grid((unsigned)gx, (unsigned)mblocks);
     const bool w4 = a.w_scale8 != nullptr;

@@ -1144,6 +1144,45 @@ def test_stream_shared_weights_and_tile_order(cuda_device, monkeypatch, weights,
     assert ((b16 - racc).abs() <= 2 * k * 2.0 ** -8 * racc.abs().max()).all()
 
 
+# stage 2 walks one, two and four column groups per workgroup (KB 4 and 2, and
+# 2 with enough M-blocks), stage 1 has 4, 2 and 3 column tiles and more than 32 M-blocks
+@pytest.mark.parametrize("weights", ["fp8", "mxfp4"])
+@pytest.mark.parametrize("bm", [16, 32])
+@pytest.mark.parametrize("H,I,keep", [(1024, 512, 37), (512, 256, 5), (4096, 256, 70),
+                                      (768, 384, 41)])
+def test_stream_m_blocks_end_with_the_metadata(cuda_device, weights, bm, H, I, keep):
+    """Stage calls given the first `keep` entries of sorted_expert_ids run the
+    first `keep` M-blocks and no other, as if num_valid_ids ended there: the
+    same a2 rows, and with one slot per token the same sums, bit for bit. Its
+    entries past `keep` are left in memory, so a block run too many shows."""
+    cfg = W.MoEConfig("short", 80 * bm, H, I, 8, 1, seed=keep, weights=weights)
+    wts = W.make_weights(cfg, device=cuda_device)
+    tw, ids = W.make_routing(cfg, device=cuda_device)
+    a1, a1s = A.per_group_quant_hip(W.make_hidden(cfg, device=cuda_device))
+    st1, st2 = ((A.moe_stage1_a8w4, A.moe_stage2_a8w4) if weights == "mxfp4" else
+                (A.moe_stage1_fp8_blockscale, A.moe_stage2_fp8_blockscale))
+    sid, sw, seid, nv, acc = A.moe_sorting(ids, tw, 8, H, torch.float32, bm)
+    assert nv[0].item() > keep * bm
+    short = torch.tensor([keep * bm, cfg.tokens], dtype=torch.int32, device=cuda_device)
+    done = sid[: keep * bm] & 0xFFFFFF
+    done = done[done < cfg.tokens].long()
+    rest = torch.ones(cfg.tokens, dtype=torch.bool, device=cuda_device)
+    rest[done] = False
+    out = {}
+    for name, e, n in (("short", seid[:keep], nv), ("ref", seid, short)):
+        a2, a2s = st1(a1, a1s, wts["w1"], wts["w1_scale"], sid, e, n, 1, bm, True)
+        y = torch.zeros_like(acc)
+        # rows that no block of this call wrote are anything: 0, for both
+        a2.view(torch.uint8)[rest] = 0
+        a2s[rest] = 0
+        st2(a2, a2s, wts["w2"], wts["w2_scale"], sid, sw, e, n, y, bm, True)
+        out[name] = a2.view(torch.uint8), a2s, y
+    for got, want in zip(out["short"], out["ref"]):
+        assert torch.equal(got, want)
+    y = out["short"][2]
+    assert torch.count_nonzero(y[rest]) == 0 and (y[done].abs().amax(1) > 0).all()
+
+
 @pytest.mark.parametrize("H", [256, 1792, 2048, 2304, 4096, 7168])
 @pytest.mark.parametrize("prequant", [False, True])   # bf16 and fp32 per-pair rows
 def test_slot_sum_wave_spans(cuda_device, H, prequant):
