@@ -103,6 +103,22 @@ __device__ __forceinline__ int a_slot(int p) {
     return W4 ? (p < 4 ? 2 * p : 2 * (p - 4) + 1) : p;
 }
 
+// Columns [n0, n0 + cols) of the per-pair rows of sorted rows [srow0, srow0 +
+// rows) set to zero.
+__device__ __forceinline__ void clear_rows(const Args& g, int srow0, int rows,
+                                           int tokens, int n0, int cols) {
+    const int esz = g.part_dtype == DT_FP32 ? 4 : 2;
+    const int pieces = cols * esz / 16;
+    for (int q = threadIdx.x; q < rows * pieces; q += kThreads) {
+        const uint32_t id = (uint32_t)g.sorted_ids[srow0 + q / pieces];
+        const int t = (int)(id & 0xFFFFFFu), s = (int)(id >> 24);
+        const int64_t pair = (int64_t)t * g.topk + s;
+        if (t >= tokens || s >= g.topk || pair >= g.a_rows) continue;
+        reinterpret_cast<v4i*>(reinterpret_cast<uint8_t*>(g.part) +
+                               (pair * g.N + n0) * esz)[q % pieces] = v4i{0, 0, 0, 0};
+    }
+}
+
 // Raw buffer resource over [base, base + bytes): loads take a 32-bit lane
 // offset plus a wave-uniform K-step offset, and read 0 past the end.
 __device__ __forceinline__ __amdgpu_buffer_rsrc_t rsrc(const void* base, int64_t bytes) {
@@ -263,8 +279,15 @@ __global__ __launch_bounds__(kThreads, 2) void moe_gemm_prefill_kernel(Args g) {
     const int r0 = tid < BM ? tid : 0;
     const uint32_t id = (uint32_t)g.sorted_ids[srow0 + r0];
     const float route_w = g.sorted_w ? g.sorted_w[srow0 + r0] : 1.0f;
-    if (e < 0 || e >= g.E) return;
     const int n0 = nt * ntw * TROWS;                     // first column of the first tile
+    if (e < 0 || e >= g.E) {
+        // an expert without weights (a mask with more experts set than w holds)
+        // adds nothing, but the slot sum reads its pairs' rows: zeros
+        if constexpr (STAGE == 2) {
+            if (g.part) clear_rows(g, srow0, BM, tokens, n0, ntw * TROWS);
+        }
+        return;
+    }
 
     int any_valid = 0;
     if (tid < BM) {

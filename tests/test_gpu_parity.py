@@ -94,6 +94,37 @@ def test_sorting_chunk_size_invariant(cuda_device, monkeypatch, ct):
     assert torch.count_nonzero(buf).item() == 0
 
 
+@pytest.mark.parametrize("weights", ["fp8", "mxfp4"])
+@pytest.mark.parametrize("prequant", [False, True])   # bf16 and fp32 per-pair rows
+@pytest.mark.parametrize("bm", [16, 64, 128])
+def test_mask_with_more_experts_than_weights(cuda_device, weights, prequant, bm):
+    """An expert_mask that sets more experts than the weights hold: the ones
+    past the weights add nothing, on per-pair rows as on the accumulator. The
+    workspace comes from memory that held NaN, so a row that is summed but
+    never written shows."""
+    cfg = W.MoEConfig("over", 400, 1024, 256, 4, 3, seed=bm, weights=weights)
+    wts = W.make_weights(cfg, device=cuda_device)
+    x = W.make_hidden(cfg, device=cuda_device)
+    tw, _ = W.make_routing(cfg, device=cuda_device)
+    g = torch.Generator().manual_seed(bm)
+    ids = torch.rand(400, 8, generator=g).argsort(1)[:, :3].to(torch.int32).to(cuda_device)
+    kw = dict(w1_scale=wts["w1_scale"], w2_scale=wts["w2_scale"], block_size_M=bm)
+    if prequant:
+        x, kw["a1_scale"] = A.per_group_quant_hip(x)
+
+    def run(mask):
+        junk = [torch.full((n,), float("nan"), device=cuda_device) for n in (1 << 22, 1 << 23)]
+        del junk
+        return W.run_layer(weights, x, wts["w1"], wts["w2"], tw, ids, **kw,
+                           expert_mask=torch.tensor(mask, dtype=torch.int32, device=cuda_device))
+
+    got, want = run([1] * 8), run([1] * 4 + [0] * 4)
+    assert torch.count_nonzero(want).item() > 0
+    # on the accumulator a token's three terms may add in another order
+    tol = 0 if bm >= 64 else 4 * 2.0 ** -8
+    assert ((got.float() - want.float()).abs() <= tol * want.float().abs().max()).all()
+
+
 # both sides of every limit of the one-bit-per-pair sort: words of 32 pairs,
 # 2048 pairs in one workgroup, 256 and 512 experts, its LDS table, one thread's
 # second pair; block sizes that divide by 1 and by the largest; chunks of the
