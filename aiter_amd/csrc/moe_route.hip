@@ -150,6 +150,10 @@ __global__ __launch_bounds__(64 * kWaves) void moe_route_kernel(Args g) {
     const int64_t lrow = live ? row : g.M - 1;
     const int E = g.E, k = g.k;
     const float NEG = -__builtin_inff();
+    // ungrouped rows come here only with few experts (lanes16)
+    constexpr bool kUngrouped = LPR == 16 && V <= 8;
+    const bool softmax = kUngrouped && g.mode == SOFTMAX;
+    const bool sigmoid = kUngrouped && g.mode == SIGMOID;
 
     float x[V];
 #pragma unroll
@@ -161,13 +165,13 @@ __global__ __launch_bounds__(64 * kWaves) void moe_route_kernel(Args g) {
     // score s (what the weight is taken from) and ranking key per expert
     float s[V], key[V];
     float m = NEG;
-    if (g.mode == SOFTMAX || (g.mode == GROUPED && g.softmax_scores)) {
+    if (softmax || (g.mode == GROUPED && g.softmax_scores)) {
         float lm = NEG;
 #pragma unroll
         for (int j = 0; j < V; ++j) lm = __builtin_fmaxf(lm, x[j]);
         m = row_max<LPR>(lm);
     }
-    if (g.mode == SOFTMAX || g.mode == SIGMOID) {
+    if (softmax || sigmoid) {
 #pragma unroll
         for (int j = 0; j < V; ++j) key[j] = x[j];
     } else {
@@ -257,9 +261,9 @@ __global__ __launch_bounds__(64 * kWaves) void moe_route_kernel(Args g) {
             }
         row_argmax<LPR>(v, i);
         float w;
-        if (g.mode == SOFTMAX) {
+        if (softmax) {
             w = expf(v - m);
-        } else if (g.mode == SIGMOID) {
+        } else if (sigmoid) {
             w = sigmoid_f32(v);
         } else {
             // the unbiased score of expert i, from its owner
@@ -278,7 +282,7 @@ __global__ __launch_bounds__(64 * kWaves) void moe_route_kernel(Args g) {
     }
 
     float scale = 1.0f;
-    if (g.mode == SOFTMAX) {
+    if (softmax) {
         if (g.need_renorm) {
             if (sum_sel != 0.0f) scale = 1.0f / sum_sel;
         } else {
@@ -289,7 +293,7 @@ __global__ __launch_bounds__(64 * kWaves) void moe_route_kernel(Args g) {
             const float Z = sum_sel + row_sum<LPR>(rest);
             if (Z != 0.0f) scale = 1.0f / Z;
         }
-    } else if (g.mode != SIGMOID) {
+    } else if (!sigmoid) {
         scale = g.need_renorm ? g.scaling / sum_sel : g.scaling;
     }
 #pragma unroll
@@ -593,6 +597,36 @@ static bool wave_groups(int64_t E, int64_t n_group) {
     return E == 64 * wave_v(E) && n_group >= 1 && n_group <= 32 && 64 % n_group == 0;
 }
 
+// Ungrouped rows that 16 lanes take faster than a wave: many rows of few
+// experts, whose 64 lanes are mostly empty. Measured on MI355X, launches back
+// to back in a graph, us on 16 lanes / on the wave (bf16, top-8):
+//   E = 8, top-2, any mode: T=4096 3.0 / 2.6, T=8192 3.2 / 3.3, T=16384 4.1 / 4.7;
+//   softmax over the whole row, whose second pass of exponentials a wave's lanes
+//   pay for however few experts they hold: E = 64 T=14336 9.4 / 9.0, T=16384
+//   9.4 / 9.9, T=65536 30.0 / 31.9; E = 72 T=32768 20.5 / 20.9, T=65536 36.7 /
+//   38.8; E = 96 T=32768 21.1 / 20.9, T=65536 37.7 / 38.3; E = 128 T=65536 37.5 /
+//   38.5, but 39.3 / 39.2 with fp32 logits and top-4 faster on the wave;
+//   softmax over the chosen: E = 64 T=32768 15.8 / 15.7, T=65536 27.9 / 28.2,
+//   T=131072 51.9 / 53.1; E = 72 and up level;
+//   sigmoid: E = 64 T=65536 28.7 / 27.2.
+static bool lanes16(int64_t M, int64_t E, int mode, int need_renorm) {
+    if (E <= 16) return M >= 8192;
+    if (mode != SOFTMAX) return false;
+    if (need_renorm) return E <= 64 && M >= 65536;
+    return E <= 64 ? M >= 16384 : E <= 96 && M >= 65536;
+}
+
+// Grouped rows of whole lanes that 16 lanes take faster: softmax scores, one or
+// two groups of 64 experts (a lane holds one expert and the groups cost the
+// general kernel little). us on 16 lanes / on the wave, top-4: one group T=10240
+// 7.8 / 7.2, T=12288 7.9 / 8.1, T=16384 8.9 / 9.8, T=65536 26.8 / 30.8; two groups
+// T=12288 8.0 / 8.0, T=16384 9.5 / 9.6, T=65536 28.2 / 30.6; four groups T=65536
+// 32.9 / 30.9.
+static bool lanes16_grouped(int64_t M, int64_t E, int64_t n_group, int mode, int softmax_scores) {
+    return mode == GROUPED && softmax_scores && E == 64 && n_group <= 2 &&
+           M >= (n_group == 1 ? 12288 : 16384);
+}
+
 }  // namespace route
 
 bool route_supported(int64_t E, int64_t k) {
@@ -628,11 +662,10 @@ void launch_moe_route(const void* gating, int dtype, int64_t M, int64_t E, int64
     const dim3 block(64 * route::kWaves);
     const dim3 g16((unsigned)ceil_div(M, 4 * route::kWaves));
     const dim3 g64((unsigned)ceil_div(M, route::kWaves));
-    // One row per wave with ballot-picked ranks, for every row but two kinds:
-    // groups that are not whole lanes, and many rows of a few experts, whose
-    // 64 lanes would be mostly empty (E = 8, top-2: T=4096 3.0 us on 16 lanes
-    // per row, 2.6 on the wave; T=8192 3.2 and 3.3; T=16384 4.1 and 4.7).
-    if (grouped ? route::wave_groups(E, n_group) : !(E <= 16 && M >= 8192)) {
+    // one row per wave with ballot-picked ranks, where the row suits it
+    if (grouped ? route::wave_groups(E, n_group) && !route::lanes16_grouped(M, E, n_group, mode,
+                                                                            softmax_scores)
+                : !route::lanes16(M, E, mode, need_renorm)) {
         g.vec = g.gs % 4 == 0 && reinterpret_cast<uintptr_t>(gating) % 16 == 0;
         auto go = [&](auto v) {
             constexpr int V = decltype(v)::value;

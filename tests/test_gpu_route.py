@@ -208,6 +208,31 @@ def test_route_row_edges(cuda_device, M, E, k, dtype):
         np.testing.assert_allclose(gw[r], p / p.sum(), rtol=2e-6, atol=0)
 
 
+# both sides of the row counts at which rows of few experts go to 16 lanes
+@pytest.mark.parametrize("M,E,k,renorm", [
+    (16383, 64, 8, False), (16384, 64, 8, False), (16385, 17, 3, False), (65535, 96, 4, False),
+    (65537, 96, 4, False), (65535, 64, 2, True), (65536, 64, 2, True)])
+def test_route_many_rows_of_few_experts(cuda_device, M, E, k, renorm):
+    x = _logits(M, E, torch.bfloat16, M + E, cuda_device)
+    w = torch.empty(M, k, dtype=torch.float32, device=cuda_device)
+    ids = torch.empty(M, k, dtype=torch.int32, device=cuda_device)
+    tei = torch.empty(M, k, dtype=torch.int32, device=cuda_device)
+    A.topk_softmax(w, ids, tei, x, renorm)
+    rw, rids, rtei = RR.topk_softmax_ref(_np(x.float()), k, renorm)
+    assert np.array_equal(_np(ids), rids) and np.array_equal(_np(tei), rtei)
+    np.testing.assert_allclose(_np(w), rw, rtol=2e-6, atol=1e-9)
+
+
+@pytest.mark.parametrize("M,n_group,topk_group", [(12287, 1, 1), (12288, 1, 1), (16383, 2, 1),
+                                                  (16385, 2, 1), (16384, 4, 2)])
+def test_grouped_many_rows_of_64_experts(cuda_device, M, n_group, topk_group):
+    x = _logits(M, 64, torch.float32, M, cuda_device)
+    w = torch.empty(M, 6, dtype=torch.float32, device=cuda_device)
+    ids = torch.empty(M, 6, dtype=torch.int32, device=cuda_device)
+    A.grouped_topk(x, w, ids, n_group, topk_group, True, True, 1.5)
+    _check_grouped(_np(x), w, ids, 6, n_group, topk_group, True, True, 1.5, None)
+
+
 @pytest.mark.parametrize("E,n_group,topk_group", [
     (64, 1, 1), (64, 32, 5), (128, 2, 1), (192, 4, 2), (256, 16, 16), (320, 8, 3), (384, 8, 4),
     (512, 32, 9), (768, 4, 3), (1024, 8, 4), (448, 8, 4), (96, 3, 2), (60, 4, 2)])
