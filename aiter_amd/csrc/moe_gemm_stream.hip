@@ -101,6 +101,7 @@ struct Args {
     int eid_shift;
     int gx;                    // stage 1: column tiles x ksplit; stage 2: 256-column groups
     int mblocks;               // M-blocks that sorted_eids has an entry for and the grid covers
+    int share;                 // the kernel form with SHARE (see launch)
     // direct M-blocks, for a layer too small to be worth a sorting launch:
     // with dir_ids set, M-block p holds routing pair p = token * topk + slot
     // of dir_tokens tokens in its first row (the rest is padding), its expert
@@ -173,7 +174,10 @@ struct Step {
 // down GEMM accumulated into acc; STAGE 3: both for one 128-wide slice of
 // the intermediate dim per workgroup (the fused layer).
 // ACC32: stage 2 adds into an fp32 accumulator (else bf16 / fp16, acc_dtype).
-template <int BM, int STAGE, bool SHUFFLED, bool W4, int D, bool XQ = false, bool ACC32 = true>
+// SHARE: M-blocks of one expert may be neighbours and then load its weights
+// through the caches; without it every M-block streams its own.
+template <int BM, int STAGE, bool SHUFFLED, bool W4, int D, bool SHARE, bool XQ = false,
+          bool ACC32 = true>
 __global__ __launch_bounds__(kThreads) void moe_gemm_stream_kernel(Args g) {
     constexpr int NRT = BM / 16;
     constexpr bool G1 = STAGE != 2;                      // runs the gate+up GEMM
@@ -222,7 +226,7 @@ __global__ __launch_bounds__(kThreads) void moe_gemm_stream_kernel(Args g) {
         e = g.dir_ids[mb];
     } else {
         e = g.sorted_eids[mb >> g.eid_shift];
-        if constexpr (!FUSED) {
+        if constexpr (SHARE) {
             ep = g.sorted_eids[max(mb - 1, 0) >> g.eid_shift];
             en = g.sorted_eids[min(mb + 1, mv - 1) >> g.eid_shift];
         }
@@ -561,7 +565,7 @@ __global__ __launch_bounds__(kThreads) void moe_gemm_stream_kernel(Args g) {
         epilogue2(jt);
     }
     };
-    if (shared_w)
+    if (SHARE && shared_w)
         k_loop(std::false_type{});
     else
         k_loop(std::true_type{});
@@ -851,16 +855,25 @@ static void launch_depth(int KB, dim3 grid, const Args& a, hipStream_t s) {
     constexpr int DM = max_depth<BM>();
     auto go = [&](auto depth) {
         constexpr int D = decltype(depth)::value;
-        if constexpr (STAGE == 2) {
-            if (a.acc_dtype != DT_FP32) {
-                hipLaunchKernelGGL(
-                    (moe_gemm_stream_kernel<BM, STAGE, SHUFFLED, W4, D, XQ, false>), grid,
-                    dim3(kThreads), 0, s, a);
-                return;
+        auto run = [&](auto share) {
+            constexpr bool SHARE = decltype(share)::value;
+            if constexpr (STAGE == 2) {
+                if (a.acc_dtype != DT_FP32) {
+                    hipLaunchKernelGGL(
+                        (moe_gemm_stream_kernel<BM, STAGE, SHUFFLED, W4, D, SHARE, XQ, false>),
+                        grid, dim3(kThreads), 0, s, a);
+                    return;
+                }
             }
-        }
-        hipLaunchKernelGGL((moe_gemm_stream_kernel<BM, STAGE, SHUFFLED, W4, D, XQ>), grid,
-                           dim3(kThreads), 0, s, a);
+            hipLaunchKernelGGL((moe_gemm_stream_kernel<BM, STAGE, SHUFFLED, W4, D, SHARE, XQ>),
+                               grid, dim3(kThreads), 0, s, a);
+        };
+        if constexpr (STAGE == 3 || XQ)
+            run(std::false_type{});
+        else if (a.share)
+            run(std::true_type{});
+        else
+            run(std::false_type{});
     };
     // One-token MXFP4 stage 1 (XQ: A from LDS, so a step holds only weight
     // fragments, 16 bytes per lane and column tile) keeps 8 steps in flight.
@@ -899,12 +912,16 @@ static void launch_bm(int bm, int KB, dim3 grid, const Args& a, hipStream_t s) {
         AMD_CHECK(false, "streaming GEMM block_m must be 16 or 32");
 }
 
-// gx column tiles (x K ranges) by mblocks M-blocks.
+// gx column tiles (x K ranges) by mblocks M-blocks. An expert has two M-blocks
+// only where the layer has more tokens than a block rows (a token that names an
+// expert twice aside, whose blocks then stream its weights each for itself);
+// below, the kernel form that looks for no neighbour and holds one K loop.
 template <int STAGE>
 static void launch(int bm, int KB, int64_t gx, int64_t mblocks, Args a, int shuffled,
                    hipStream_t s) {
     a.gx = (int)gx;
     a.mblocks = (int)mblocks;
+    a.share = (STAGE == 2 ? a.a_rows / a.topk : a.a_rows) > bm;
     AMD_CHECK(gx * mblocks < (int64_t(1) << 31), "too many M-blocks");
     const dim3 grid((unsigned)gx, (unsigned)mblocks);
     const bool w4 = a.w_scale8 != nullptr;
