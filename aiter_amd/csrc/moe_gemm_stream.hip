@@ -146,18 +146,27 @@ __device__ __forceinline__ void tile_of(int L, int gx, int mv, int& bx, int& mb)
 // K weight bytes per group, so its setup and epilogue weigh more the fewer
 // groups it walks; but the walk has to leave most CUs a workgroup, and the last
 // of the ~512 that run at a time should not be nearly empty. Measured on MI355X
-// (layer, us, at one / two / four groups; mv M-blocks): fp8, 16 K steps, 16
-// groups: mv 101 431 / 424 / 420, mv 160 678 / 666 / 666, mv 219 873 / 848 /
-// 874; 3 steps: mv 122 112 / 110 / 111; 6 steps, 12 groups: mv 101 127 / 132 /
-// 136, mv 250 281 / 280 / 280; 2 steps, 28 groups: mv 18 45.9 / 43.4 / 44.5, mv
-// 250 248 / 238 / 235. MXFP4, 16 steps: mv 160 363 / 370 / 354, mv 250 528 /
-// 540 / 517, skewed routing at T=64 142 / 147 / 163.
+// (layer, us, at one / two / four groups; mv M-blocks):
+//   1 and 2 steps: 16 groups fp8 mv 8 26.6 / 27.5 / 29.9, mv 42 42.7 / 43.8 / 45.0,
+//   mv 56 48.9 / 47.7 / 48.8, MXFP4 mv 8 23.1 / 23.4 / 25.8, mv 42 33.5 / 33.9 /
+//   34.9; 28 groups fp8 mv 35 48.3 / 47.0 / 47.6, mv 62 78.8 / 78.5 / 77.1, mv 160
+//   178.6 / 173.3 / 172.4, MXFP4 mv 160 121.6 / 113.4 / 111.7;
+//   fp8, 3 steps: mv 122 112 / 110 / 111; 6 steps, 12 groups: mv 101 127 / 132 /
+//   136, mv 250 281 / 280 / 280; 16 steps, 16 groups: mv 101 431 / 424 / 420, mv
+//   160 678 / 666 / 666, mv 219 873 / 848 / 874;
+//   MXFP4, 16 steps: mv 160 363 / 370 / 354, mv 250 528 / 540 / 517, skewed routing
+//   at T=64 142 / 147 / 163.
+// The lines between these points are not each measured on both sides, and the
+// MXFP4 ones only at 2 and 16 steps. Over 1 to 16 steps, both weight types, 1 to
+// 200 tokens and both routings the choice is within 3% of the best of the three
+// in most cases; the largest losses found are 8%, at skewed routing (fp8, 16
+// steps, T=128: four groups 335 us, one 311).
 template <bool W4>
 __device__ __forceinline__ int walk_groups(int mv, int groups, int KB) {
     const bool two = (groups & 1) == 0 && 2 * KB <= kMaxKB;
     const bool four = (groups & 3) == 0 && 4 * KB <= kMaxKB;
     const int w2 = mv * groups / 2, w4 = w2 / 2;           // workgroups
-    if (KB <= 2) return four && w4 >= 256 ? 4 : two ? 2 : 1;
+    if (KB <= 2) return four && w4 >= 256 ? 4 : two && w2 >= 448 ? 2 : 1;
     if (W4) return four && w4 >= 600 ? 4 : 1;
     if (four && KB >= 8 && w4 >= 384 && w4 <= 512) return 4;
     return two && (w2 >= 3 * 512 || (w2 >= 384 && (w2 & 511) >= 256)) ? 2 : 1;

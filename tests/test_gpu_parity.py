@@ -1175,12 +1175,12 @@ def test_stream_shared_weights_and_tile_order(cuda_device, monkeypatch, weights,
     assert ((b16 - racc).abs() <= 2 * k * 2.0 ** -8 * racc.abs().max()).all()
 
 
-# stage 2 walks one, two and four column groups per workgroup (KB 4 and 2, and
-# 2 with enough M-blocks), stage 1 has 4, 2 and 3 column tiles and more than 32 M-blocks
+# stage 2 walks one, two and four column groups per workgroup (two K steps and 5,
+# 60 and 70 M-blocks), stage 1 has 4, 2 and 3 column tiles and more than 32 M-blocks
 @pytest.mark.parametrize("weights", ["fp8", "mxfp4"])
 @pytest.mark.parametrize("bm", [16, 32])
-@pytest.mark.parametrize("H,I,keep", [(1024, 512, 37), (512, 256, 5), (4096, 256, 70),
-                                      (768, 384, 41)])
+@pytest.mark.parametrize("H,I,keep", [(1024, 512, 37), (512, 256, 5), (4096, 256, 60),
+                                      (4096, 256, 70), (768, 384, 41)])
 def test_stream_m_blocks_end_with_the_metadata(cuda_device, weights, bm, H, I, keep):
     """Stage calls given the first `keep` entries of sorted_expert_ids run the
     first `keep` M-blocks and no other, as if num_valid_ids ended there: the
