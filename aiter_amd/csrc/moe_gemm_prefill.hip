@@ -280,7 +280,7 @@ __global__ __launch_bounds__(kThreads, 2) void moe_gemm_prefill_kernel(Args g) {
     const uint32_t id = (uint32_t)g.sorted_ids[srow0 + r0];
     const float route_w = g.sorted_w ? g.sorted_w[srow0 + r0] : 1.0f;
     const int n0 = nt * ntw * TROWS;                     // first column of the first tile
-    if (e < 0 || e >= g.E) {
+    if (__builtin_expect(e < 0 || e >= g.E, 0)) {
         // an expert without weights (a mask with more experts set than w holds)
         // adds nothing, but the slot sum reads its pairs' rows: zeros
         if constexpr (STAGE == 2) {
