@@ -194,7 +194,7 @@ static void stage1_dispatch(const uint8_t* a, const float* sa, int64_t sa_row, i
 }
 
 // Stage 2 runs on the prefill kernel for this shape (the only stage-2
-// kernel that can also write per-pair bf16 rows instead of accumulating).
+// kernel that can also write per-pair rows, bf16 or fp32, instead of accumulating).
 static bool stage2_on_prefill(int64_t bm, int64_t I, int64_t H, WScale w2s, int64_t a_rows,
                               int64_t E, int64_t est_pairs) {
     return !(stream_supported(bm, I) && H % 256 == 0) && prefill_supported(bm, I) &&
@@ -309,17 +309,40 @@ struct FusedLayout {
 
 int64_t align256(int64_t x) { return (x + 255) & ~int64_t(255); }
 
-// Layers that sum in fp32 throughout (see fused_entry): per-pair fp32 rows
-// written and read once, or fp32 atomics, which go past the XCDs' L2s and meet
-// on a token's row. Layer times on MI355X, hidden 4096, top-8, atomics / rows:
-// 16 experts of inter 1536 T=256 163 / 152 us, T=1500 429 / 394, T=8192 2030 /
-// 1900; 32 of 256 experts of inter 2048 T=2048 213 / 195, T=8192 397 / 361; all
-// 256 T=600 1231 / 1252, T=2048 1414 / 1433, T=8192 2907 / 2878. Beyond this
-// many bytes of rows the workspace would outgrow the layer's other sections,
-// so larger layers keep the accumulator.
+// Whether a layer that sums in fp32 throughout (see fused_entry) writes per-pair
+// fp32 rows, stored and read once, instead of fp32 atomics on the accumulator.
+// Atomics go past the XCDs' L2s and meet on a token's row, but hide behind the
+// weights that stage 2 streams where experts have few rows; rows cost a second
+// pass. Layer times on MI355X, hidden 4096, top-8, us with atomics / rows:
+//   256 experts of inter 2048 T=600 1248 / 1271, T=1200 1283 / 1317, T=2048 1375 /
+//   1406, T=3000 1522 / 1534, T=4096 1777 / 1765, T=8192 2861 / 2855; of inter 512
+//   T=800 353 / 362, T=1200 389 / 382, T=2048 525 / 493;
+//   128 of inter 2048 T=600 669 / 688, T=1200 782 / 774; 64 T=400 353 / 359, T=600
+//   403 / 403, T=1200 546 / 538; 32 T=200 183 / 181, T=400 218 / 213;
+//   16 of inter 1536 T=100 77 / 74, T=1500 430 / 401; of inter 768 T=256 90 / 81;
+//   shares of 256 experts of inter 2048: 32 T=600 179 / 178, T=2048 235 / 212, T=8192
+//   466 / 422; 128 T=1000 680 / 684, T=4096 953 / 932.
+// So: a share (most of a token's rows are elsewhere, so are most of the atomics'
+// collisions, but the second pass reads an eighth or so), rows that stay in the
+// L2s, or enough rows per expert against the K range that stage 2 runs per row,
+// more of them where the rows outgrow the last-level cache.
+// The rows take topk times the accumulator's memory, in a share too, where most
+// of them are never touched. A GiB is what a call may ask for: a bound by choice,
+// not where rows stop winning (see T=8192).
 constexpr int64_t kMaxF32RowBytes = int64_t(1) << 30;
 
-bool f32_rows_fit(int64_t T, int64_t k, int64_t H) { return T * k * H * 4 <= kMaxF32RowBytes; }
+bool f32_rows(int64_t T, int64_t H, int64_t I, int64_t E_sort, int64_t E_local, int64_t k,
+              int64_t bm) {
+    const int64_t bytes = T * k * H * 4;
+    // (MXFP4 weights leave the prefill kernel below some rows per expert; the
+    // workspace, which is sized by this, does not know the weights)
+    if (bytes > kMaxF32RowBytes ||
+        !stage2_on_prefill(bm, I, H, WScale{nullptr, nullptr}, T * k, E_local, -1))
+        return false;
+    if (E_local < E_sort || bytes <= (int64_t(32) << 20)) return true;
+    const int64_t rows = T * k / E_local;
+    return rows >= 32 && rows * 1024 >= I * (bytes <= (int64_t(256) << 20) ? 36 : 64);
+}
 
 // E_local: the experts this GPU holds (E_sort: the ids' range, global under
 // an expert mask). sum32: the layer sums in fp32 throughout.
@@ -347,7 +370,7 @@ FusedLayout fused_layout(int64_t T, int64_t H, int64_t I, int64_t E_sort, int64_
     L.off_a2_scale = o;    o = align256(o + T * k * (I / 128) * 4);
     // fp32 accumulator [T, H], or per-pair rows [T*k, H] when stage 2 runs on
     // the prefill kernel: room for either
-    const int64_t row_bytes = !sum32 ? 2 : f32_rows_fit(T, k, H) ? 4 : 0;
+    const int64_t row_bytes = !sum32 ? 2 : f32_rows(T, H, I, E_sort, E_local, k, bm) ? 4 : 0;
     L.off_acc = o;         o = align256(o + std::max(T * H * 4, T * k * H * row_bytes));
     L.kcnt_bytes = L.ksplit > 1 ? align256(L.kmb * (I / 128) * 4) : 0;
     L.off_kcnt = o;        o += L.kcnt_bytes;
@@ -585,7 +608,8 @@ void fused_entry(const void* hidden_states, int hidden_dtype, const void* w1, WS
     const int part_dtype = sum32 ? DT_FP32 : DT_BF16;
     void* part = stage2_on_prefill(block_m, inter_dim, model_dim, w2s, tokens * topk, num_experts,
                                    local_pairs) &&
-                         (!sum32 || f32_rows_fit(tokens, topk, model_dim))
+                         (!sum32 || f32_rows(tokens, model_dim, inter_dim, E_sort, num_experts, topk,
+                                              block_m))
                      ? ws + L.off_acc : nullptr;
     hipStream_t s = (hipStream_t)stream;
     timing_mark(0, s);

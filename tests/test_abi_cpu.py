@@ -317,6 +317,29 @@ def test_fused_moe_is_a_registered_custom_op():
         assert out.shape == (6, 256) and out.dtype == torch.float16
 
 
+@pytest.mark.parametrize("tokens,H,I,E,G,k,bm,rows", [
+    (1500, 4096, 1536, 16, 16, 8, 64, True), (2048, 4096, 2048, 32, 256, 8, 64, True),
+    (8192, 4096, 2048, 32, 256, 8, 64, True),      # a GiB of rows
+    (8193, 4096, 2048, 32, 256, 8, 64, False),
+    (600, 4096, 2048, 256, 256, 8, 64, False), (2048, 4096, 2048, 256, 256, 8, 64, False),
+    (4096, 4096, 2048, 256, 256, 8, 64, True), (1200, 4096, 512, 256, 256, 8, 64, True),
+    (64, 4096, 1536, 16, 16, 8, 32, False),        # stage 2 on the stream kernel
+    (64, 4096, 1536, 16, 16, 8, 16, False),
+    (64, 4224, 1536, 16, 16, 8, 64, False)])       # stage 2 on the general kernel
+def test_prequant_workspace_holds_rows_only_where_they_are_written(lib, tokens, H, I, E, G, k, bm,
+                                                                   rows):
+    """The last big section of the layer on fp8 activations is the fp32 accumulator
+    [tokens, H], or per-pair fp32 rows, topk times as large, where stage 2 writes
+    them; the other sections are those of the layer that quantises, whose bf16
+    rows or accumulator are known."""
+    q = [tokens, H, I, E, G, k, bm]
+    up = lambda n: (n + 255) // 256 * 256
+    full = lib.aiter_amd_fused_moe_workspace_bytes(*q)
+    rest = full - up(tokens * H * max(4, 2 * k))
+    got = lib.aiter_amd_fused_moe_prequant_workspace_bytes(*q) - rest
+    assert got == up(tokens * H * 4 * (k if rows else 1))
+
+
 def test_fused_moe_compiles_without_a_warning():
     """fused_moe traces into one full graph of the custom op, and tracing warns
     of nothing."""

@@ -1131,6 +1131,29 @@ def test_prequant_layer_beyond_the_row_limit(cuda_device):
     assert ((a - b).abs() <= b.abs() * 2.0 ** -7 + 8 * 2.0 ** -23 * b.abs().max() * 8).all()
 
 
+@pytest.mark.parametrize("weights", ["fp8", "mxfp4"])
+def test_prequant_layer_rows_per_expert(cuda_device, weights):
+    """30 rows per expert sum on the fp32 accumulator, 35 on per-pair fp32 rows
+    (39 and 46 MB of them): the tokens they share agree, within the bound above.
+    The workspace held NaN."""
+    T, k, E, H, I = 700, 8, 160, 2048, 128
+    cfg = W.MoEConfig("rpe", T, H, I, E, k, seed=4, weights=weights)
+    wts = W.make_weights(cfg, device=cuda_device)
+    tw, ids = W.make_routing(cfg, device=cuda_device)
+    a1, a1s = A.per_group_quant_hip(W.make_hidden(cfg, device=cuda_device))
+
+    def run(n):
+        junk = torch.full((1 << 24,), float("nan"), device=cuda_device)
+        del junk
+        return W.run_layer(weights, a1[:n], wts["w1"], wts["w2"], tw[:n], ids[:n],
+                           w1_scale=wts["w1_scale"], w2_scale=wts["w2_scale"],
+                           a1_scale=a1s[:n], block_size_M=128).float()
+
+    a, b = run(T)[:600], run(600)
+    assert torch.count_nonzero(b).item() > 0
+    assert ((a - b).abs() <= b.abs() * 2.0 ** -7 + 8 * 2.0 ** -23 * b.abs().max() * 8).all()
+
+
 # column-tile counts that 8 divides and that it does not (stage 1 inter / 128,
 # stage 2 model_dim / 256 over the groups a workgroup walks), M-blocks below, at
 # and above the 32 of a whole round of groups, K-step counts of 1, 2, 3, 5, 6 and
