@@ -44,22 +44,19 @@ def _stream(dev: torch.device) -> int:
 
 # The switches that a layer call reads (AITER_AMD_*), from os.environ's own
 # table where it is there: os.environ.get of a name that is not set encodes it
-# and raises and catches a KeyError, about 1 us, and a call reads five. Both
-# see changes at once.
-_ENV_TABLE = getattr(os.environ, "_data", None)
-if not isinstance(_ENV_TABLE, dict) or (_ENV_TABLE and
-                                        not isinstance(next(iter(_ENV_TABLE)), bytes)):
-    _ENV_TABLE = None
+# and raises and catches a KeyError, about 1 us, and a call reads five. The
+# table is looked up on each call, so a change or another os.environ is seen.
 _SWITCHES = ("AITER_AMD_TUNED_FMOE", "AITER_AMD_FUSED", "AITER_AMD_ST_KSPLIT1",
              "AITER_AMD_SORT_CT")
-_SWITCH_KEYS = tuple(n.encode() for n in _SWITCHES)
+_SWITCH_KEYS = tuple(os.fsencode(n) for n in _SWITCHES)
 
 
 def _switches() -> tuple:
     """The values of _SWITCHES (None: not set), part of the cached plans' key."""
-    if _ENV_TABLE is None:
+    table = getattr(os.environ, "_data", None)
+    if type(table) is not dict or not os.supports_bytes_environ:
         return tuple(os.environ.get(n) for n in _SWITCHES)
-    get = _ENV_TABLE.get
+    get = table.get
     a, b, c, d = _SWITCH_KEYS
     return get(a), get(b), get(c), get(d)
 

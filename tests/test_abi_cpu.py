@@ -340,6 +340,26 @@ def test_prequant_workspace_holds_rows_only_where_they_are_written(lib, tokens, 
     assert got == up(tokens * H * 4 * (k if rows else 1))
 
 
+def test_layer_switches_follow_the_environment(monkeypatch):
+    """A layer's cached plan is keyed by the switches' values now: one set or taken
+    away in os.environ, and those of another mapping in its place."""
+    import os
+
+    from aiter_amd.fused_moe import _SWITCHES, _switches
+
+    text = lambda: tuple(v if v is None else os.fsdecode(v) for v in _switches())
+    for n in _SWITCHES:
+        monkeypatch.delenv(n, raising=False)
+    assert text() == (None,) * 4
+    for i, n in enumerate(_SWITCHES):
+        monkeypatch.setenv(n, str(i))
+    assert text() == ("0", "1", "2", "3")
+    monkeypatch.delenv(_SWITCHES[2])
+    assert text() == ("0", "1", None, "3")
+    monkeypatch.setattr(os, "environ", {_SWITCHES[1]: "7"})
+    assert text() == (None, "7", None, None)
+
+
 def test_fused_moe_compiles_without_a_warning():
     """fused_moe traces into one full graph of the custom op, and tracing warns
     of nothing."""
