@@ -69,6 +69,8 @@ def _layer_plan(M, model_dim, inter_dim, E, global_E, topk, block_size_M, a8w4, 
     and switch values."""
     if block_size_M not in (None, -1):
         block_m = int(block_size_M)
+        if prequant and block_m <= 0:
+            raise ValueError(f"block_size_M must be positive, got {block_m}")
     else:
         block_m = select_block_m(M, topk, E, model_dim, inter_dim, a8w4, device, global_E)
     if prequant:

@@ -360,6 +360,18 @@ def test_layer_switches_follow_the_environment(monkeypatch):
     assert text() == (None, "7", None, None)
 
 
+def test_prequant_layer_refuses_a_negative_block():
+    """fp8 activations with a negative block_size_M (but -1, which means none given)
+    raise, as when sorting was given it; the layer that quantises takes its own."""
+    from aiter_amd.fused_moe import _layer_plan, _switches
+
+    args = (40, 1024, 512, 8, 8, 2)
+    for b in (-2, -16):
+        with pytest.raises(ValueError, match="block_size_M"):
+            _layer_plan(*args, b, False, True, torch.device("cuda:0"), _switches())
+        assert _layer_plan(*args, b, False, False, torch.device("cuda:0"), _switches())[0] == b
+
+
 def test_fused_moe_compiles_without_a_warning():
     """fused_moe traces into one full graph of the custom op, and tracing warns
     of nothing."""
