@@ -1155,9 +1155,9 @@ def test_prequant_layer_rows_per_expert(cuda_device, weights):
 
 
 # column-tile counts that 8 divides and that it does not (stage 1 inter / 128,
-# stage 2 model_dim / 256 over the groups a workgroup walks), M-blocks below, at
-# and above the 32 of a whole round of groups, K-step counts of 1, 2, 3, 5, 6 and
-# 8 in stage 2, experts with one M-block and with many
+# stage 2 model_dim / 256), M-blocks below, at and above the 32 of a whole round
+# of groups, K-step counts of 1, 2, 3, 5, 6 and 8 in stage 2, experts with one
+# M-block and with many (column walks: the two tests after this one)
 @pytest.mark.parametrize("weights", ["fp8", "mxfp4"])
 @pytest.mark.parametrize("bm", [16, 32])
 @pytest.mark.parametrize("tokens,H,I,E", [
@@ -1165,8 +1165,7 @@ def test_prequant_layer_rows_per_expert(cuda_device, weights):
     (260, 512, 640, 40), (333, 2048, 768, 33), (512, 1024, 1024, 8), (90, 3584, 256, 64)])
 def test_stream_shared_weights_and_tile_order(cuda_device, monkeypatch, weights, bm, tokens, H, I,
                                               E):
-    """The stream kernel's workgroup order, column walks and weight-load
-    policies against the prefill kernels (64-row blocks), which pass the oracle
+    """The stream kernel's workgroup order and weight-load policies against the prefill kernels (64-row blocks), which pass the oracle
     tests: with the staggered K walk off both sum K blocks in the same order,
     so stage 1 is bit for bit the same and a pair's stage-2 row too; a token's
     pairs then add in any order, (k - 1) * 2^-24 of the sum of their magnitudes."""
@@ -1196,6 +1195,80 @@ def test_stream_shared_weights_and_tile_order(cuda_device, monkeypatch, weights,
     # a bf16 moe_buf rounds after every add: half a spacing, 2^-8, per pair
     b16 = got[bm, torch.bfloat16][2].float()
     assert ((b16 - racc).abs() <= 2 * k * 2.0 ** -8 * racc.abs().max()).all()
+
+
+def _walk_groups(w4, mv, groups, KB):
+    """The stream kernel's own choice of stage 2's column groups per workgroup
+    (walk_groups, moe_gemm_stream.hip), with the name of its line."""
+    two, four = groups % 2 == 0 and 2 * KB <= 64, groups % 4 == 0 and 4 * KB <= 64
+    w2 = mv * groups // 2
+    w4_ = w2 // 2
+    if KB <= 2:
+        return (4, "short") if four and w4_ >= 256 else (2, "short") if two and w2 >= 448 else \
+            (1, "short")
+    if w4:
+        return (4, "mxfp4") if four and w4_ >= 600 else (1, "mxfp4")
+    if four and KB >= 8 and 384 <= w4_ <= 512:
+        return 4, "fp8"
+    if two and w2 >= 3 * 512:
+        return 2, "fp8 many"
+    return (2, "fp8 tail") if two and w2 >= 384 and w2 & 511 >= 256 else (1, "fp8")
+
+
+# 600 pairs over 40 experts (more M-blocks than a round of 32 groups of four), K
+# ranges of 3, 6, 2, 8 and 5 steps, 16, 12, 8 and 28 column groups: walks of two
+# and four leave column counts that 8 divides and that it does not
+@pytest.mark.parametrize("weights", ["fp8", "mxfp4"])
+@pytest.mark.parametrize("bm", [16, 32])
+@pytest.mark.parametrize("H,I", [(4096, 384), (3072, 768), (2048, 384), (7168, 256), (4096, 1024),
+                                 (2048, 640)])
+def test_stream_stage2_forced_walks(cuda_device, monkeypatch, weights, bm, H, I):
+    """Stage 2 walking two and four column groups against one: with one slot per
+    token every output element has one add, so they are equal bit for bit."""
+    acc = _stage2_of(cuda_device, weights, 600, H, I, 40, bm)
+    monkeypatch.setenv("AITER_AMD_ST_NTW2", "1")
+    one, mv = acc()
+    assert mv >= 40 and torch.count_nonzero(one).item() > 0
+    for ntw in (2, 4):
+        monkeypatch.setenv("AITER_AMD_ST_NTW2", str(ntw))
+        assert torch.equal(acc()[0], one), ntw
+
+
+# one case per line of the kernel's choice
+@pytest.mark.parametrize("weights,tokens,H,I,E,want", [
+    ("fp8", 700, 4096, 256, 8, (1, "short")), ("fp8", 850, 4096, 256, 8, (2, "short")),
+    ("mxfp4", 850, 4096, 128, 8, (2, "short")), ("mxfp4", 1100, 4096, 256, 8, (4, "short")),
+    ("mxfp4", 600, 4096, 384, 8, (1, "mxfp4")), ("mxfp4", 2500, 4096, 384, 8, (4, "mxfp4")),
+    ("fp8", 1600, 4096, 1024, 8, (4, "fp8")), ("fp8", 3100, 4096, 384, 8, (2, "fp8 many")),
+    ("fp8", 750, 4096, 384, 8, (2, "fp8 tail")), ("fp8", 750, 4096, 768, 8, (2, "fp8 tail")),
+    ("fp8", 1050, 4096, 768, 8, (1, "fp8"))])
+def test_stream_stage2_own_walk(cuda_device, monkeypatch, weights, tokens, H, I, E, want):
+    monkeypatch.delenv("AITER_AMD_ST_NTW2", raising=False)
+    acc = _stage2_of(cuda_device, weights, tokens, H, I, E, 16)
+    own, mv = acc()
+    assert _walk_groups(weights == "mxfp4", mv, H // 256, I // 128) == want, mv
+    monkeypatch.setenv("AITER_AMD_ST_NTW2", "1")
+    one = acc()[0]
+    assert torch.count_nonzero(one).item() > 0 and torch.equal(own, one)
+
+
+def _stage2_of(dev, weights, tokens, H, I, E, bm):
+    """A call of stage 2 on one layer's a2, top-1: (accumulator, M-blocks)."""
+    cfg = W.MoEConfig("walks", tokens, H, I, E, 1, seed=tokens + I, weights=weights)
+    wts = W.make_weights(cfg, device=dev)
+    tw, ids = W.make_routing(cfg, device=dev)
+    a1, a1s = A.per_group_quant_hip(W.make_hidden(cfg, device=dev))
+    st1, st2 = ((A.moe_stage1_a8w4, A.moe_stage2_a8w4) if weights == "mxfp4" else
+                (A.moe_stage1_fp8_blockscale, A.moe_stage2_fp8_blockscale))
+    sid, sw, seid, nv, acc = A.moe_sorting(ids, tw, E, H, torch.float32, bm)
+    a2, a2s = st1(a1, a1s, wts["w1"], wts["w1_scale"], sid, seid, nv, 1, bm, True)
+
+    def run():
+        y = torch.zeros_like(acc)
+        st2(a2, a2s, wts["w2"], wts["w2_scale"], sid, sw, seid, nv, y, bm, True)
+        return y, nv[0].item() // bm
+
+    return run
 
 
 # stage 2 walks one, two and four column groups per workgroup (two K steps and 5,

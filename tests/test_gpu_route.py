@@ -122,7 +122,9 @@ def _check_grouped(x, w, ids, k, n_group, topk_group, renorm, softmax, scaling, 
         assert all(v <= lo + 1e-6 for v in rest), (r, gids[r], rids[r])
 
 
-@pytest.mark.parametrize("M", [37, 2000])   # whole-wave rows under 1024 tokens, 16-lane above
+# 96 experts in 3 groups are the general kernel's: a wave per row under 1024 tokens,
+# 16 lanes above
+@pytest.mark.parametrize("M", [37, 2000])
 @pytest.mark.parametrize("E,n_group,topk_group,k", [(256, 8, 4, 8), (64, 4, 2, 4), (96, 3, 1, 5)])
 @pytest.mark.parametrize("softmax,renorm,scaling", [(True, True, 1.0), (False, False, 2.5),
                                                     (False, True, 1.5)])
@@ -236,29 +238,50 @@ def test_grouped_many_rows_of_64_experts(cuda_device, M, n_group, topk_group):
 @pytest.mark.parametrize("E,n_group,topk_group", [
     (64, 1, 1), (64, 32, 5), (128, 2, 1), (192, 4, 2), (256, 16, 16), (320, 8, 3), (384, 8, 4),
     (512, 32, 9), (768, 4, 3), (1024, 8, 4), (448, 8, 4), (96, 3, 2), (60, 4, 2)])
-@pytest.mark.parametrize("mode", ["softmax", "biased"])
+@pytest.mark.parametrize("mode", ["softmax", "sigmoid", "biased"])
 def test_grouped_forms(cuda_device, E, n_group, topk_group, mode):
     """Every lanes-per-group form of the one-row-per-wave kernel, and groups
-    that are not whole lanes (the general kernel), against the oracle."""
-    k = min(8, topk_group * (E // n_group))
-    x = _logits(41, E, torch.float32, E + n_group, cuda_device)
-    bias = None
+    that are not whole lanes (the general kernel), against the oracle: ids and
+    weights of every rank."""
+    _grouped_against_oracle(cuda_device, 41, E, n_group, topk_group, mode)
+
+
+# one experts-per-lane form of the general kernel each: under 1024 rows a wave per
+# row up to 64, 128, 256, 512 and 1024 experts, from there on 16 lanes up to 16, 64,
+# 128 and 256 experts
+@pytest.mark.parametrize("M", [41, 1030])
+@pytest.mark.parametrize("E,n_group,topk_group", [(12, 2, 1), (60, 4, 2), (96, 3, 1), (160, 8, 4),
+                                                  (448, 8, 4), (640, 8, 3)])
+@pytest.mark.parametrize("mode", ["softmax", "sigmoid", "biased"])
+def test_grouped_general_kernel(cuda_device, M, E, n_group, topk_group, mode):
+    _grouped_against_oracle(cuda_device, M, E, n_group, topk_group, mode)
+
+
+@pytest.mark.parametrize("E,n_group,topk_group", [
+    (64, 1, 1), (64, 32, 5), (128, 2, 1), (192, 4, 2), (256, 16, 16), (320, 8, 3), (384, 8, 4),
+    (512, 32, 9), (768, 4, 3), (1024, 8, 4), (448, 8, 4), (96, 3, 2), (60, 4, 2), (160, 8, 4)])
+def test_biased_grouped_switched_off_experts(cuda_device, E, n_group, topk_group):
+    """A bias of -inf takes an expert out: never chosen while the kept groups
+    hold others, of which every rank's id and weight is checked."""
+    per = E // n_group
+    k = min(8, topk_group * (per - (per + 4) // 5))
+    bias = (torch.randn(E, generator=torch.Generator().manual_seed(E)) * 0.3).to(cuda_device)
+    bias[::5] = float("-inf")
+    ids = _grouped_against_oracle(cuda_device, 41, E, n_group, topk_group, "biased", bias, k)
+    assert (ids % 5 != 0).all()
+
+
+def _grouped_against_oracle(dev, M, E, n_group, topk_group, mode, bias=None, k=None):
+    k = k or min(8, topk_group * (E // n_group))
+    x = _logits(M, E, torch.float32, E + n_group, dev)
+    w = torch.empty(M, k, dtype=torch.float32, device=dev)
+    ids = torch.empty(M, k, dtype=torch.int32, device=dev)
     if mode == "biased":
-        bias = (torch.randn(E, generator=torch.Generator().manual_seed(E)) * 0.3).to(cuda_device)
-        bias[::5] = float("-inf")                                   # experts switched off
-    w = torch.empty(41, k, dtype=torch.float32, device=cuda_device)
-    ids = torch.empty(41, k, dtype=torch.int32, device=cuda_device)
-    if bias is None:
-        A.grouped_topk(x, w, ids, n_group, topk_group, True, True, 1.5)
-    else:
+        if bias is None:
+            bias = (torch.randn(E, generator=torch.Generator().manual_seed(E)) * 0.3).to(dev)
         A.biased_grouped_topk(x, bias, w, ids, n_group, topk_group, True, 1.5)
-    if E // n_group < 2:
-        return                                  # a group of one has no second choice to sum
-    if bias is not None and k > 2:
-        k = 2                                   # ranks that every kept group set still fills
-        w, ids = w[:, :k], ids[:, :k]
-        rw, rids = RR.grouped_topk_ref(_np(x), k, n_group, topk_group, False, False, 1.0, _np(bias))
-        assert (_np(ids) == rids).all(axis=1).mean() >= 0.97        # at most one row on a tie
-        return
-    _check_grouped(_np(x), w, ids, k, n_group, topk_group, True, True, 1.5,
+    else:
+        A.grouped_topk(x, w, ids, n_group, topk_group, True, mode == "softmax", 1.5)
+    _check_grouped(_np(x), w, ids, k, n_group, topk_group, True, mode == "softmax", 1.5,
                    None if bias is None else _np(bias))
+    return ids
