@@ -608,8 +608,8 @@ void fused_entry(const void* hidden_states, int hidden_dtype, const void* w1, WS
     const int part_dtype = sum32 ? DT_FP32 : DT_BF16;
     void* part = stage2_on_prefill(block_m, inter_dim, model_dim, w2s, tokens * topk, num_experts,
                                    local_pairs) &&
-                         (!sum32 || f32_rows(tokens, model_dim, inter_dim, E_sort, num_experts, topk,
-                                              block_m))
+                         (!sum32 || f32_rows(tokens, model_dim, inter_dim, E_sort, num_experts,
+                                             topk, block_m))
                      ? ws + L.off_acc : nullptr;
     hipStream_t s = (hipStream_t)stream;
     timing_mark(0, s);

@@ -117,9 +117,9 @@ struct Args {
     int xq_bf16;
 };
 
-// Workgroup L (x fastest) of the grid -> (column tile, M-block), L on XCD L % 8. Where 8
-// divides the gx column tiles, column by column: XCD x then runs tiles x, x + 8,
-// ... of every M-block, and M-blocks of one expert meet its weights in one L2.
+// Workgroup L (x fastest) of the grid -> (column tile, M-block), L on XCD L % 8.
+// Where 8 divides the gx column tiles, column by column: XCD x then runs tiles x,
+// x + 8, ... of every M-block, and M-blocks of one expert meet its weights in one L2.
 // Otherwise XCD x takes groups of four consecutive M-blocks (the groups x, x +
 // 8, ...) through all their column tiles, the M-blocks of a group side by side,
 // and the last mv % 32 of the mv valid M-blocks go column by column, so that
@@ -470,8 +470,10 @@ __global__ __launch_bounds__(kThreads) void moe_gemm_stream_kernel(Args g) {
     };
 
     // The K loop, a copy for weights that this M-block alone reads (non-temporal
-    // loads: they should displace nothing) and one for weights it shares with
-    // the expert's other M-blocks. Measured on MI355X, MiMo dims: with
+    // loads: they should displace nothing) and, with SHARE, one for weights it
+    // shares with the expert's other M-blocks (both copies and the neighbours' ids
+    // cost a layer that has none: hidden 7168, inter 256, 257 experts, T=4 51.0 us,
+    // 47.4 with one copy). Measured on MI355X, MiMo dims: with
     // non-temporal loads throughout, blocks of one expert each read its weights
     // from HBM (skewed routing, 16-row blocks, T=256: 610 us, 428 with the two
     // copies); with ordinary loads throughout, uniform routing T=256 ran 1163
@@ -506,8 +508,8 @@ __global__ __launch_bounds__(kThreads) void moe_gemm_stream_kernel(Args g) {
     // different offsets of their weight rows
     // (M-blocks that share weights walk in step, so that one's loads are the
     // others' L2 hits)
-    const int krot =
-        G1 && g.krot ? D * (int)(((unsigned)bx * 5u + (unsigned)(ONCE ? mb : e) * 3u) % (KBS / D)) : 0;
+    const unsigned stagger = (unsigned)bx * 5u + (unsigned)(ONCE ? mb : e) * 3u;
+    const int krot = G1 && g.krot ? D * (int)(stagger % (KBS / D)) : 0;
     auto km = [&](int k) {
         int r = k - kbeg + krot;
         if (r >= KBS) r -= KBS;

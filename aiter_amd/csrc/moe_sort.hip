@@ -23,9 +23,9 @@
 // sorts a small batch; larger ones are cut into chunks of `ct` tokens, a
 // workgroup each. Up to 512 experts and 2048 pairs (of the batch or chunk) the
 // workgroup's LDS table holds one bit per (expert, pair) (the moe_sort_*bits
-// kernels below). Beyond, it is a bitmap table[token][expert] of slot masks (a byte per cell for topk <= 8, a u32
-// up to topk 32, so duplicates of an expert inside one token's top-k are all
-// kept, in slot order); a thread per expert then counts the expert's pairs
+// kernels below). Beyond, it is a bitmap table[token][expert] of slot masks (a
+// byte per cell for topk <= 8, a u32 up to topk 32, so duplicates of an expert
+// inside one token's top-k are all kept, in slot order); a thread per expert then counts the expert's pairs
 // in each group of 8 rows (1 for u32 cells) into an LDS prefix, and a thread
 // per pair writes the pair at its segment's start + the expert's pairs in
 // earlier chunks + in earlier row groups + in earlier bits of its own group
@@ -931,8 +931,8 @@ bool launch_moe_sort(const int32_t* topk_ids, const float* topk_w, const int32_t
         const size_t lds = bit_lds((int)E, (int)(rows * topk));
         const int64_t side = zero_blocks + p.q_blocks;
         auto go = [&](auto kern, int nt) {
-            hipLaunchKernelGGL(kern, dim3(1 + (unsigned)ceil_div(side, nt / kSortThreads)), dim3(nt),
-                               lds, stream, p);
+            hipLaunchKernelGGL(kern, dim3(1 + (unsigned)ceil_div(side, nt / kSortThreads)),
+                               dim3(nt), lds, stream, p);
         };
         if (E > 256)
             go(moe_sort_bits_kernel<1024, 8>, 1024);

@@ -307,7 +307,8 @@ void launch_slot_sum(const void* part, int part_dtype, const int32_t* topk_ids,
     const bool per_wave = mask != nullptr;
     const int64_t spans = ceil_div(cols, 64 * 64 / (part_dtype == DT_FP32 ? 4 : 2));
     const int blocks =
-        (int)std::min<int64_t>(per_wave ? ceil_div(rows * spans, 4) : rows, per_wave ? 65536 : 8192);
+        (int)(per_wave ? std::min<int64_t>(ceil_div(rows * spans, 4), 65536)
+                       : std::min<int64_t>(rows, 8192));
     auto go = [&](auto kern, auto* rows_of_pairs) {
         hipLaunchKernelGGL(kern, dim3(blocks), dim3(256), 0, stream, rows_of_pairs, topk_ids, mask,
                            (int)num_experts, num_valid, (uint16_t*)out, rows, (int)topk,

@@ -1,6 +1,7 @@
 // 1 x 128 FP8 quantisation of one 256-thread block's 16 groups: the body of
 // per_group_quant_fp8_kernel, shared with the sorting launch (which runs it
-// in extra blocks at decode sizes; `tid` is the thread within the 256). Semantics: quant.hip's header.
+// in extra blocks at decode sizes; `tid` is the thread within the 256).
+// Semantics: quant.hip's header.
 #pragma once
 #include "common.h"
 
