@@ -1045,19 +1045,18 @@ __global__ __launch_bounds__(kThreads) void moe_token_stage2_kernel(TokArgs g) {
     const int nsl = wv < g.topk ? (g.topk - wv + kWaves - 1) / kWaves : 0;
     const int nsteps = nsl * KB;          // a multiple of D (D divides KB)
 
+    // a slot routed outside [0, E) contributes nothing: stage 1 wrote no a2 row for
+    // it and its weight may be anything, so its sum is dropped whole (fold_slot)
+    auto slot_ok = [&](int eraw) { return eraw >= 0 && eraw < g.E; };
     // step q: slot wv + 4 (q / KB), K block q % KB; eraw is that slot's expert
     // id, fetched a slot ahead so that no weight load waits on it
     auto load = [&](TokStep<W4>& st, int q, int eraw) __attribute__((always_inline)) {
         const int sl = wv + kWaves * (q / KB);
         const int kb = q - (q / KB) * KB;
-        const bool ok = eraw >= 0 && eraw < g.E;
-        const int e = ok ? eraw : 0;
+        const int e = slot_ok(eraw) ? eraw : 0;
         const uint8_t* ap = g.a2 + (int64_t)sl * I + kb * 128 + (W4 ? lq * 16 : lq * 32);
-        const v4i a0 = *reinterpret_cast<const v4i*>(ap);
-        const v4i a1 = *reinterpret_cast<const v4i*>(ap + AHI);
-        // a slot routed outside [0, E) contributes nothing: zero operands
-        st.a[0] = ok ? a0 : v4i{0, 0, 0, 0};
-        st.a[1] = ok ? a1 : v4i{0, 0, 0, 0};
+        st.a[0] = *reinterpret_cast<const v4i*>(ap);
+        st.a[1] = *reinterpret_cast<const v4i*>(ap + AHI);
         const uint8_t* we = g.w2 + (int64_t)e * g.H * KBY;
 #pragma unroll
         for (int ct = 0; ct < 2; ++ct) {
@@ -1130,11 +1129,11 @@ __global__ __launch_bounds__(kThreads) void moe_token_stage2_kernel(TokArgs g) {
         }
     };
     // a slot's K blocks are done: weight its sum into the row
-    auto fold_slot = [&](float rw) __attribute__((always_inline)) {
+    auto fold_slot = [&](float rw, bool ok) __attribute__((always_inline)) {
 #pragma unroll
         for (int ct = 0; ct < 2; ++ct) {
 #pragma unroll
-            for (int v = 0; v < 4; ++v) row[ct][v] += pacc[ct][v] * rw;
+            for (int v = 0; v < 4; ++v) row[ct][v] += ok ? pacc[ct][v] * rw : 0.0f;
             pacc[ct] = v4f{0.f, 0.f, 0.f, 0.f};
         }
     };
@@ -1147,6 +1146,7 @@ __global__ __launch_bounds__(kThreads) void moe_token_stage2_kernel(TokArgs g) {
         int jl = 0;                         // slot of the steps being loaded
         int el = slot_id(0), en = slot_id(1);
         float rw = slot_w(0);               // weight of the slot being computed
+        bool ok = slot_ok(el);
         load_e8(e8c, 0, el);
 #pragma unroll
         for (int d = 0; d < D; ++d) load(buf[d], d, el);
@@ -1171,13 +1171,14 @@ __global__ __launch_bounds__(kThreads) void moe_token_stage2_kernel(TokArgs g) {
                     for (int d = 0; d < D; ++d) e8c[ct][d] = e8n[ct][d];
             }
             if (slot_end) {
-                fold_slot(rw);
+                fold_slot(rw, ok);
                 rw = slot_w(jl);
+                ok = slot_ok(el);
             }
         }
 #pragma unroll
         for (int d = 0; d < D; ++d) compute(buf[d], d);
-        fold_slot(rw);
+        fold_slot(rw, ok);
     }
     // output row 0 sits in lanes lq == 0, element 0: column lr of each tile
     if (lq == 0) {

@@ -1132,6 +1132,45 @@ def test_prequant_layer_beyond_the_row_limit(cuda_device):
 
 
 @pytest.mark.parametrize("weights", ["fp8", "mxfp4"])
+@pytest.mark.parametrize("prequant", [False, True])
+@pytest.mark.parametrize("inter", [384, 1024])     # stage-2 depths 1 and 8
+def test_fused_moe_direct_ids_out_of_range(cuda_device, monkeypatch, weights, prequant, inter):
+    """One token some of whose slots name no expert (what routing gives past its
+    last candidate, with any weight): they add nothing, as on the sorted layer,
+    whatever the workspace held. Without the staggered K walk the two differ in
+    the order of the fp32 sum alone: one bf16 rounding."""
+    monkeypatch.setenv("AITER_AMD_ST_ROT", "0")
+    monkeypatch.setenv("AITER_AMD_ST_KSPLIT1", "1")   # one K range: direct M-blocks
+    k = 6
+    cfg = W.MoEConfig("oor", 1, 1024, inter, 8, k, seed=inter, weights=weights)
+    wts = W.make_weights(cfg, device=cuda_device)
+    x = W.make_hidden(cfg, device=cuda_device)
+    kw = dict(w1_scale=wts["w1_scale"], w2_scale=wts["w2_scale"], block_size_M=16)
+    if prequant:
+        x, kw["a1_scale"] = A.per_group_quant_hip(x)
+    nan = float("nan")
+    cases = [([3, -1, 5, 8, 0, 0x7fffffff], [0.5, nan, 0.25, nan, 0.125, nan]),
+             ([-1, 2, -1, -1, 8, 7], [nan, 0.5, 1.0, nan, float("inf"), 0.25]),
+             ([-1] * k, [nan] * k)]
+
+    def run(ids, tw, direct):
+        monkeypatch.setenv("AITER_AMD_DIRECT", direct)
+        junk = torch.full((1 << 22,), nan, device=cuda_device)
+        del junk
+        return W.run_layer(weights, x, wts["w1"], wts["w2"],
+                           torch.tensor([tw], device=cuda_device),
+                           torch.tensor([ids], dtype=torch.int32, device=cuda_device), **kw)
+
+    for ids, tw in cases:
+        got, ref = run(ids, tw, "1"), run(ids, tw, "0")
+        assert torch.isfinite(ref).all()
+        assert (torch.count_nonzero(ref).item() > 0) == (max(i for i in ids if i < 8) >= 0)
+        a, b = got.float(), ref.float()
+        tol = 2.0 ** -7 * torch.maximum(a.abs(), b.abs()) + k * 2.0 ** -23 * b.abs().max() * 8
+        assert ((a - b).abs() <= tol).all(), ids     # (the last term: where terms cancel)
+
+
+@pytest.mark.parametrize("weights", ["fp8", "mxfp4"])
 def test_prequant_layer_rows_per_expert(cuda_device, weights):
     """30 rows per expert sum on the fp32 accumulator, 35 on per-pair fp32 rows
     (39 and 46 MB of them): the tokens they share agree, within the bound above.
