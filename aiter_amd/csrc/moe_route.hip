@@ -299,7 +299,7 @@ __global__ __launch_bounds__(64 * kWaves) void moe_route_kernel(Args g) {
 #pragma unroll
     for (int t = 0; t < kMaxK; ++t) {
         if (t >= k) break;
-        if (lane == t && live) {
+        if (lane == t % LPR && live) {                  // top-17 and up: more ranks than 16 lanes
             g.w[row * g.ws + t] = sel_v[t] * scale;
             g.ids[row * g.is + t] = sel_i[t];
             if (g.tei) g.tei[row * k + t] = (int32_t)((int64_t)t * g.M + row);

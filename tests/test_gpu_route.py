@@ -225,6 +225,35 @@ def test_route_many_rows_of_few_experts(cuda_device, M, E, k, renorm):
     np.testing.assert_allclose(_np(w), rw, rtol=2e-6, atol=1e-9)
 
 
+# more ranks than a row has lanes, on 16 lanes (the last sizes of each form) and not
+@pytest.mark.parametrize("M", [41, 1030, 16390])
+@pytest.mark.parametrize("E,k", [(64, 17), (60, 32), (40, 31)])
+@pytest.mark.parametrize("mode", ["softmax", "sigmoid", "grouped softmax", "grouped biased"])
+def test_route_more_than_16_ranks(cuda_device, M, E, k, mode):
+    x = _logits(M, E, torch.float32, M + E + k, cuda_device)
+    w = torch.full((M, k), -7.0, dtype=torch.float32, device=cuda_device)
+    ids = torch.full((M, k), -7, dtype=torch.int32, device=cuda_device)
+    if mode == "softmax":
+        tei = torch.full((M, k), -7, dtype=torch.int32, device=cuda_device)
+        A.topk_softmax(w, ids, tei, x, False)
+        rw, rids, rtei = RR.topk_softmax_ref(_np(x), k, False)
+        assert np.array_equal(_np(tei), rtei)
+    elif mode == "sigmoid":
+        A.topk_sigmoid(w, ids, x)
+        rw, rids = RR.topk_sigmoid_ref(_np(x), k)
+    else:
+        bias = None
+        if mode == "grouped biased":
+            bias = (torch.randn(E, generator=torch.Generator().manual_seed(E)) * 0.3).to(cuda_device)
+            A.biased_grouped_topk(x, bias, w, ids, 2, 2, True, 1.5)
+        else:
+            A.grouped_topk(x, w, ids, 2, 2, True, True, 1.5)
+        return _check_grouped(_np(x), w, ids, k, 2, 2, True, bias is None, 1.5,
+                              None if bias is None else _np(bias))
+    assert np.array_equal(_np(ids), rids)
+    np.testing.assert_allclose(_np(w), rw, rtol=2e-6, atol=1e-9)
+
+
 @pytest.mark.parametrize("M,n_group,topk_group", [(12287, 1, 1), (12288, 1, 1), (16383, 2, 1),
                                                   (16385, 2, 1), (16384, 4, 2)])
 def test_grouped_many_rows_of_64_experts(cuda_device, M, n_group, topk_group):
