@@ -318,7 +318,9 @@ int aiter_amd_fused_moe_a8w4(const void* hidden_states, int hidden_dtype, const 
                              int64_t workspace_bytes, void* stream);
 
 /* Bytes of workspace for aiter_amd_fused_moe_prequant; arguments as
- * aiter_amd_fused_moe_workspace_bytes. */
+ * aiter_amd_fused_moe_workspace_bytes. Per-pair fp32 rows, where stage 2 may
+ * write them (at most 1 GiB), take topk times the memory of the fp32
+ * accumulator that other layers use. */
 int64_t aiter_amd_fused_moe_prequant_workspace_bytes(int64_t tokens, int64_t model_dim,
                                                      int64_t inter_dim, int64_t num_experts,
                                                      int64_t global_experts, int64_t topk,
